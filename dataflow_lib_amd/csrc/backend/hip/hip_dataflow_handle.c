@@ -138,6 +138,16 @@ static int hip_register_native_code(Dataflow_Handle * dataflow_handle, char * na
 			(void) hipGetLastError();
 		}
 
+		static const char * const variant_suffixes[HIP_NUM_VARIANTS] = HIP_VARIANT_SUFFIXES;
+		for (int v = 0; v < HIP_NUM_VARIANTS; v++) {
+			char variant_sym[FUNC_SYMBOL_MAX_LEN + 16];
+			snprintf(variant_sym, sizeof(variant_sym), "%s%s", sym, variant_suffixes[v]);
+			if (hipModuleGetFunction(&f.variant_handles[v], *module, variant_sym) != hipSuccess) {
+				f.variant_handles[v] = NULL;
+				(void) hipGetLastError();
+			}
+		}
+
 		memcpy(&f.op_skeleton, &func_op_skeletons[i], sizeof(Op_Skeleton));
 		f.hip_external_func = NULL;
 		f.op_extra = NULL;
@@ -258,6 +268,14 @@ static int hip_submit_op(Dataflow_Handle * dataflow_handle, Op * op, int stream_
 		if (cfg.gridDimX == 0 || cfg.gridDimY == 0 || cfg.gridDimZ == 0) {
 			return 0;
 		}
+		hipFunction_t kernel = f->function_handle;
+		if (cfg.variant != 0) {
+			kernel = cfg.variant <= HIP_NUM_VARIANTS ? f->variant_handles[cfg.variant - 1] : NULL;
+			if (!kernel) {
+				fprintf(stderr, "hip backend: op %s: the launch configuration chose kernel variant %u, which the code object lacks\n", nick, cfg.variant);
+				return -1;
+			}
+		}
 		Hip_Context * hc = (Hip_Context *) dataflow_handle->ctx;
 		if (f->function_config.shares_module_scratch && hc->two_pass_stream != HIP_NO_STREAM && hc->two_pass_stream != stream_id) {
 			/* the previous op using the module scratch ran on another stream:
@@ -269,7 +287,7 @@ static int hip_submit_op(Dataflow_Handle * dataflow_handle, Op * op, int stream_
 			HIP_CHECK_RET(hipEventRecord(hc->two_pass_event, prev), -1, "ordering op %s after the previous scratch user", nick);
 			HIP_CHECK_RET(hipStreamWaitEvent(stream, hc->two_pass_event, 0), -1, "ordering op %s after the previous scratch user", nick);
 		}
-		if (launch(f->function_handle, &cfg, stream, op)) {
+		if (launch(kernel, &cfg, stream, op)) {
 			fprintf(stderr, "hip backend: op %s: kernel launch failed\n", nick);
 			return -1;
 		}

@@ -350,8 +350,7 @@ int softmax_set_attribute_config(Dataflow_Handle * dataflow_handle, Hip_Function
 	return 0;
 }
 
-/* one workgroup per row; small rows get a smaller workgroup */
-static int smx_config(Hip_Launch_Config * c, Dataflow_Handle * h, Hip_Function * f, int n_rows, int n_cols, const char * what) {
+static int smx_config(Hip_Launch_Config * c, Dataflow_Handle * h, Hip_Function * f, int n_rows, int n_cols, const void * x, const void * out, const char * what) {
 	const size_t elem = arg_elem_bytes(f, 2);
 	if (n_rows < 0 || n_cols < 0 || elem == 0) {
 		fprintf(stderr, "Error: %s: invalid shape (%d x %d) or dtype...\n", what, n_rows, n_cols);
@@ -359,6 +358,16 @@ static int smx_config(Hip_Launch_Config * c, Dataflow_Handle * h, Hip_Function *
 	}
 	if (n_rows == 0 || n_cols == 0) {
 		set_1d(c, 0, 1, 0);
+		return 0;
+	}
+	const int kernel = is_fp8(f, 2) ? SMX_MAIN : smx_kernel_for(n_rows, n_cols, (int) elem, ptr_bits(x), ptr_bits(out));
+	if (kernel != SMX_MAIN) {
+		/* all rows at once: a workgroup of the row's waves, or
+		 * SMX_ROWS_PER_WG rows of one wave each */
+		const int waves = smx_rows_waves(kernel == SMX_ROWS ? SMX_ROWS_CH : SMX_WIDE_ROWS_CH, n_rows, n_cols, (int) elem, ptr_bits(x), ptr_bits(out));
+		if (waves == 1) set_1d(c, (unsigned) MY_CEIL(n_rows, SMX_ROWS_PER_WG), 64 * SMX_ROWS_PER_WG, 0);
+		else set_1d(c, (unsigned) n_rows, (unsigned) (64 * waves), 0);
+		c->variant = kernel == SMX_ROWS ? HIP_VARIANT_ROWS : HIP_VARIANT_WIDE_ROWS;
 		return 0;
 	}
 	/* persistent over rows: one workgroup of SMX_THREADS per CU (a row fills
@@ -370,7 +379,7 @@ static int smx_config(Hip_Launch_Config * c, Dataflow_Handle * h, Hip_Function *
 
 int softmax_set_launch_config(Hip_Launch_Config * hip_launch_config, Dataflow_Handle * dataflow_handle, Hip_Function * hip_function, Op * op) {
 	const int n_rows = ARG(op, 0, int), n_cols = ARG(op, 1, int);
-	if (smx_config(hip_launch_config, dataflow_handle, hip_function, n_rows, n_cols, "softmax")) return -1;
+	if (smx_config(hip_launch_config, dataflow_handle, hip_function, n_rows, n_cols, ARG(op, 2, void *), ARG(op, 3, void *), "softmax")) return -1;
 	/* fp8 logits: long rows keep smx_config's one SMX_THREADS workgroup per CU
 	 * (the next row prefetched into LDS); other rows that fit the registers
 	 * take two smaller workgroups per CU */
@@ -387,7 +396,8 @@ int softmax_cross_entropy_loss_set_launch_config(Hip_Launch_Config * hip_launch_
 		fprintf(stderr, "Error: softmax cross entropy loss: mean_loss needs the per-row loss buffer...\n");
 		return -1;
 	}
-	return smx_config(hip_launch_config, dataflow_handle, hip_function, ARG(op, 0, int), ARG(op, 1, int), "softmax cross entropy loss");
+	return smx_config(hip_launch_config, dataflow_handle, hip_function, ARG(op, 0, int), ARG(op, 1, int), ARG(op, 2, void *), ARG(op, 2, void *),
+					  "softmax cross entropy loss");
 }
 
 int cross_entropy_loss_set_launch_config(Hip_Launch_Config * hip_launch_config, Dataflow_Handle * dataflow_handle, Hip_Function * hip_function, Op * op) {

@@ -7,5 +7,6 @@
 #include "rope.hip"
 #include "swiglu.hip"
 #include "softmax_xent.hip"
+#include "softmax_rows.hip"
 #include "gather_scatter.hip"
 #include "fp8_ops.hip"

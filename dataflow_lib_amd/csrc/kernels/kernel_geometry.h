@@ -37,6 +37,13 @@
  * other SMX_MAXCH - SMX_PF chunks of the next row are prefetched into VGPRs */
 #define SMX_PF 9
 
+/* softmax / cross-entropy, "_rows" kernels: rows held by 1..16 waves,
+ * SMX_ROWS_CH 16-byte chunks per thread; a row that one wave holds shares its
+ * workgroup with SMX_ROWS_PER_WG - 1 others */
+#define SMX_ROWS_CH 8
+#define SMX_WIDE_ROWS_CH 16
+#define SMX_ROWS_PER_WG 4
+
 /* RoPE, head_dim <= 512. Vector path: one ROPE_SLOT_THREADS workgroup per
  * token at a time (persistent over tokens, next token prefetched), thread t
  * owning Q chunks t + 256 j (j < ROPE_QJ) and K chunks t + 256 j (j < ROPE_KJ)
@@ -173,6 +180,56 @@ GEOM_FN int f8_smx_pf_ok(int n_cols) {
 
 GEOM_FN int f8_smx_regs_ok(int n_cols) {
 	return n_cols > 0 && (n_cols % 8) == 0 && n_cols / 8 <= F8_SMX_CH * F8_SMX_THREADS;
+}
+
+/* softmax "_rows" kernels: the 16-byte chunks a row's window can have
+ * (SmxWindow), or 0 when input and output lie differently within a chunk */
+GEOM_FN int smx_rows_chunks(int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
+	const long bytes = (long) n_cols * elem_bytes;
+	const unsigned long long line = ((x ^ out) & 127ull) ? 15ull : 127ull;
+	if (((x ^ out) & 15ull) != 0ull || ((x | out) % (unsigned) elem_bytes) != 0ull) return 0;
+	const long slack = ((bytes & (long) line) | (long) (x & line)) ? (long) line : 0;
+	return (int) ((bytes + slack + 15) / 16);
+}
+
+/* Waves per row for a kernel of ch chunks per thread, or 0 when 16 waves do
+ * not hold the row. */
+GEOM_FN int smx_rows_waves(int ch, int n_rows, int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
+	const int chunks = smx_rows_chunks(n_cols, elem_bytes, x, out);
+	if (chunks == 0 || chunks > 16 * 64 * ch) return 0;
+	int g = (chunks + 64 * ch - 1) / (64 * ch);
+	/* few rows: more waves each, until the chip has 8 per CU */
+	while (g <= 8 && (long) n_rows * g < 2048 && chunks > 64 * g) g *= 2;
+	return g;
+}
+
+/* Which kernel a softmax / cross-entropy call takes. In order:
+ * - SMX_ROWS (8 chunks per thread) while the row needs at most 8 waves (16-bit)
+ *   or 4 (fp32), so that at least two rows share a CU, and up to 16 waves when
+ *   no two rows have to share one (16 x 50257 bf16: 9.4 us, wide 11.7);
+ * - SMX_WIDE_ROWS (16 chunks) up to twice that: 1024 x 50257 bf16 41.4 us
+ *   against 50.7 with 13 waves of 8 chunks, of which a CU holds one workgroup;
+ *   fp32 8192 x 16384 184.2 against 199.9;
+ * - rows of more than 8192 chunks, and fp32 rows of more than 6144 when there
+ *   are many of them, go to the main kernel, which overlaps one row with the
+ *   next on the same CU (1024 x 100000 bf16 78.5 us, wide 98.3; 4096 x 32000
+ *   fp32 169.4, wide 184.1), unless they are unaligned, which it does not
+ *   hold in registers (1024 x 128257 bf16 557 us, wide 116).
+ */
+#define SMX_MAIN 0
+#define SMX_ROWS 1
+#define SMX_WIDE_ROWS 2
+#define SMX_FEW_ROWS 256   /* no more rows than CUs: each row has a CU to itself */
+GEOM_FN int smx_kernel_for(int n_rows, int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
+	const int chunks = smx_rows_chunks(n_cols, elem_bytes, x, out);
+	const int few = n_rows <= SMX_FEW_ROWS;
+	/* the main kernel holds the row in registers too */
+	const int main_regs = ((x | out) & 15ull) == 0ull && ((long) n_cols * elem_bytes) % 16 == 0;
+	if (chunks == 0 || chunks > 1024 * SMX_WIDE_ROWS_CH) return SMX_MAIN;
+	if (chunks <= 1024 * SMX_ROWS_CH && (few || chunks <= (elem_bytes < 4 ? 512 : 256) * SMX_ROWS_CH)) return SMX_ROWS;
+	if (!main_regs) return SMX_WIDE_ROWS;
+	if (elem_bytes == 4 && chunks > 6144 && n_rows >= 8 * SMX_FEW_ROWS) return SMX_MAIN;
+	return chunks <= 1024 * SMX_ROWS_CH ? SMX_WIDE_ROWS : SMX_MAIN;
 }
 
 /* RoPE vector path: tokens per workgroup step. fp8 rows are half as long as

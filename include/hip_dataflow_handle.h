@@ -68,7 +68,18 @@ typedef struct hip_launch_config {
 	unsigned int blockDimY;
 	unsigned int blockDimZ;
 	unsigned int sharedMemBytes;
+	/* which of the op's kernels to launch: 0 function_handle, i > 0
+	 * variant_handles[i - 1] */
+	unsigned int variant;
 } Hip_Launch_Config;
+
+/* Further kernels of an op, with the same parameters, for shapes that its main
+ * kernel is not the best for: "<symbol>" + suffix in the code object, chosen
+ * by the launch configuration. */
+#define HIP_VARIANT_ROWS 1        /* "_rows" */
+#define HIP_VARIANT_WIDE_ROWS 2   /* "_wide_rows" */
+#define HIP_NUM_VARIANTS 2
+#define HIP_VARIANT_SUFFIXES {"_rows", "_wide_rows"}
 
 typedef struct hip_function Hip_Function;
 
@@ -86,6 +97,8 @@ struct hip_function {
 	 * Used by ops whose cross-workgroup reduction is finished deterministically
 	 * in a second pass. NULL when absent. */
 	hipFunction_t finish_function_handle;
+	/* NULL where the code object has none */
+	hipFunction_t variant_handles[HIP_NUM_VARIANTS];
 	Hip_Set_Launch_Config set_finish_launch_config;
 
 	/* external functions */

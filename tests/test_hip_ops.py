@@ -728,6 +728,55 @@ def special_logits(dt, shape, seed):
     return to_storage(x, dt)
 
 
+# (rows, columns, elements the tensors start off a 128-byte line): around the
+# lengths where a row takes another wave, another kernel or the element path
+# (16-bit: 4096 columns per wave, 32768 and 65536 per kernel, 131072; fp32
+# half), short rows that share a workgroup, and more rows than one group of
+# the loss sum counts
+ROW_SHAPES = [(9, 2047, 0), (9, 2049, 1), (5, 4088, 0), (5, 4097, 3), (7, 16385, 0), (5, 32761, 1), (5, 32776, 0), (3, 65529, 5),
+              (3, 65544, 8), (2, 131001, 0), (2, 131073, 1), (259, 40001, 0), (2051, 200, 0), (523, 65, 7)]
+
+
+@pytest.mark.parametrize("dt", DTS, ids=dt_id)
+@pytest.mark.parametrize("shape", ROW_SHAPES, ids=lambda s: "%dx%d+%d" % s)
+def test_softmax_rows_of_any_alignment(hdl, dt, shape):
+    """Softmax and the fused loss on rows whose 16-byte chunks reach into the
+    rows beside them: every output, and the elements before and after the
+    tensor untouched."""
+    from dataflow_lib_amd import api
+    n_rows, n_cols, off = shape
+    es, pad = (4 if dt == FP32 else 2), 64
+    X = logits(dt, (n_rows, n_cols), seed=161)
+    labels = rng(162).integers(0, n_cols, size=n_rows).astype(np.uint32)
+    labels[0], labels[-1] = 0, n_cols - 1
+    pre, lo, hi = (np.empty((n_rows, n_cols)) for _ in range(3))
+    loss, mean = np.empty(n_rows), np.zeros(1)
+    assert oracle().oracle_softmax(dt, dt, n_rows, n_cols, ptr(X), ptr(pre)) == 0
+    assert oracle().oracle_softmax_cross_entropy(dt, n_rows, n_cols, ptr(X), ptr(labels), ptr(lo), ptr(hi), ptr(loss), ptr(mean)) == 0
+    store = X.dtype
+    guard = np.full(n_rows * n_cols + 2 * pad, 7, store)
+
+    def inside(buf, what):
+        a = buf[pad + off:pad + off + X.size]
+        assert (buf[:pad + off] == 7).all() and (buf[pad + off + X.size:] == 7).all(), what
+        return a.reshape(X.shape)
+
+    with Dev(hdl) as d:
+        px = d.put(X, off * es)
+        po = d.put(guard) + (pad + off) * es
+        assert api.submit_softmax(hdl, 0, dt, dt, n_rows, n_cols, px, po) == 0
+        out = inside(d.get(po - (pad + off) * es, guard.shape, store), "softmax wrote outside its rows")
+        check_rounded(out, dt, pre, what="softmax")
+        full = guard.copy()
+        full[pad + off:pad + off + X.size] = X.ravel()
+        pi, pl, ploss, pmean = d.put(full), d.put(labels), d.empty(4 * n_rows), d.empty(4)
+        assert api.submit_softmax_cross_entropy_loss(hdl, 0, dt, n_rows, n_cols, pi + (pad + off) * es, pl, ploss, pmean) == 0
+        out = inside(d.get(pi, full.shape, store), "fused loss wrote outside its rows")
+        check_rounded(out, dt, lo, hi, what="fused dlogits")
+        check_f32(d.get(ploss, (n_rows,), np.float32), loss, rel=1e-4, what="fused loss")
+        check_f32(d.get(pmean, (1,), np.float32), mean, rel=1e-4, what="fused mean loss")
+
+
 # more rows than workgroups (each walks 2-3 rows with the next row, its label
 # and labelled logit in flight); 32000 and 24576 + 8 columns leave a partial
 # last chunk, 128256 is the Llama-3 vocabulary
