@@ -361,7 +361,7 @@ static int smx_config(Hip_Launch_Config * c, Dataflow_Handle * h, Hip_Function *
 		return 0;
 	}
 	const int kernel = is_fp8(f, 2) ? SMX_MAIN : smx_kernel_for(n_rows, n_cols, (int) elem, ptr_bits(x), ptr_bits(out));
-	if (kernel != SMX_MAIN) {
+	if (kernel == SMX_ROWS || kernel == SMX_WIDE_ROWS) {
 		/* all rows at once: a workgroup of the row's waves, or
 		 * SMX_ROWS_PER_WG rows of one wave each */
 		const int waves = smx_rows_waves(kernel == SMX_ROWS ? SMX_ROWS_CH : SMX_WIDE_ROWS_CH, n_rows, n_cols, (int) elem, ptr_bits(x), ptr_bits(out));
@@ -374,6 +374,7 @@ static int smx_config(Hip_Launch_Config * c, Dataflow_Handle * h, Hip_Function *
 	 * its VGPRs and half its LDS) */
 	const long grid = MY_MIN((long) n_rows, (long) dev(h)->cu_count);
 	set_1d(c, (unsigned) grid, SMX_THREADS, 0);
+	if (kernel == SMX_LONG_ROWS) c->variant = HIP_VARIANT_LONG_ROWS;
 	return 0;
 }
 

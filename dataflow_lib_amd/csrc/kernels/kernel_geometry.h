@@ -36,6 +36,9 @@
 /* chunks per thread of the next row prefetched into LDS (9 x 16 KB); the
  * other SMX_MAXCH - SMX_PF chunks of the next row are prefetched into VGPRs */
 #define SMX_PF 9
+/* "_long_rows" kernels (16-bit): the same with more chunks per thread, the
+ * next row's chunks past SMX_PF loaded at the top of their own row */
+#define SMX_LONG_MAXCH 20
 
 /* softmax / cross-entropy, "_rows" kernels: rows held by 1..16 waves,
  * SMX_ROWS_CH 16-byte chunks per thread; a row that one wave holds shares its
@@ -89,8 +92,10 @@
 
 #ifdef __HIPCC__
 #define GEOM_FN __host__ __device__ __forceinline__
+#define GEOM_CONST constexpr GEOM_FN
 #else
 #define GEOM_FN static inline
+#define GEOM_CONST GEOM_FN
 #endif
 
 /* RMSNorm: 16-byte chunks per row, or 0 when the element path must be used */
@@ -182,6 +187,12 @@ GEOM_FN int f8_smx_regs_ok(int n_cols) {
 	return n_cols > 0 && (n_cols % 8) == 0 && n_cols / 8 <= F8_SMX_CH * F8_SMX_THREADS;
 }
 
+/* softmax register-row paths: the fewest chunks per thread that a row there
+ * has (smx_kernel_for sends shorter ones elsewhere) */
+GEOM_CONST int smx_regs_atleast(int elem_bytes, int maxch) {
+	return maxch > SMX_MAXCH ? SMX_MAXCH + 1 : (elem_bytes == 4 ? 6 : 8);
+}
+
 /* softmax "_rows" kernels: the 16-byte chunks a row's window can have
  * (SmxWindow), or 0 when input and output lie differently within a chunk */
 GEOM_FN int smx_rows_chunks(int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
@@ -204,6 +215,7 @@ GEOM_FN int smx_rows_waves(int ch, int n_rows, int n_cols, int elem_bytes, unsig
 }
 
 /* Which kernel a softmax / cross-entropy call takes. In order:
+ * - SMX_LONG_ROWS for aligned 16-bit rows of 17 to 20 chunks per thread;
  * - SMX_ROWS (8 chunks per thread) while the row needs at most 8 waves (16-bit)
  *   or 4 (fp32), so that at least two rows share a CU, and up to 16 waves when
  *   no two rows have to share one (16 x 50257 bf16: 9.4 us, wide 11.7);
@@ -219,12 +231,14 @@ GEOM_FN int smx_rows_waves(int ch, int n_rows, int n_cols, int elem_bytes, unsig
 #define SMX_MAIN 0
 #define SMX_ROWS 1
 #define SMX_WIDE_ROWS 2
+#define SMX_LONG_ROWS 3
 #define SMX_FEW_ROWS 256   /* no more rows than CUs: each row has a CU to itself */
 GEOM_FN int smx_kernel_for(int n_rows, int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
 	const int chunks = smx_rows_chunks(n_cols, elem_bytes, x, out);
 	const int few = n_rows <= SMX_FEW_ROWS;
 	/* the main kernel holds the row in registers too */
 	const int main_regs = ((x | out) & 15ull) == 0ull && ((long) n_cols * elem_bytes) % 16 == 0;
+	if (main_regs && elem_bytes < 4 && chunks > 1024 * SMX_MAXCH && ((long) n_cols * elem_bytes) / 16 <= 1024 * SMX_LONG_MAXCH) return SMX_LONG_ROWS;
 	if (chunks == 0 || chunks > 1024 * SMX_WIDE_ROWS_CH) return SMX_MAIN;
 	if (chunks <= 1024 * SMX_ROWS_CH && (few || chunks <= (elem_bytes < 4 ? 512 : 256) * SMX_ROWS_CH)) return SMX_ROWS;
 	if (!main_regs) return SMX_WIDE_ROWS;

@@ -318,6 +318,12 @@ __device__ __forceinline__ float chunk_max(const R16 & r, float m) {
 /* waits for every outstanding vector-memory access of this wave
  * (s_waitcnt vmcnt(0); expcnt and lgkmcnt left at their maxima) */
 #define WAIT_VMEM_ALL() __builtin_amdgcn_s_waitcnt(0x0F70)
+/* waits until at most N remain outstanding */
+template <int N>
+__device__ __forceinline__ void wait_vmem() {
+	static_assert(N < 64, "six bits");
+	__builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
 /* waits for every outstanding LDS access of this wave (lgkmcnt(0)) */
 #define WAIT_LDS_ALL() __builtin_amdgcn_s_waitcnt(0xC07F)
 
@@ -337,9 +343,17 @@ typedef __attribute__((address_space(3))) void * lds_ptr_t;
  * workgroup barrier guards the buffer, and the reductions' barriers wait for
  * LDS only: the one wait for memory in a row comes after its output
  * stores. */
-template <typename T, typename TO, bool FUSED>
+template <typename T, typename TO, bool FUSED, int MAXCH = SMX_MAXCH>
 __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO * out, const uint32_t * labels, float * loss) {
 	constexpr int VEC = VecOf<T>::N;
+	/* chunks per thread that every row here has: shorter ones go to other
+	 * kernels (smx_kernel_for). The first MINCH chunks go without a test of
+	 * the row's count, so those tests' masks need not be kept in (spilled)
+	 * scalar registers: bf16 fused 1024 x 100000 91.5 -> 87.1 us, softmax
+	 * 1024 x 128256 98.2 -> 95.7 us. Not in the kernels that then spilled
+	 * vector registers (fp16 softmax, and the bf16 ones of 20 chunks). */
+	constexpr int ATLEAST = smx_regs_atleast((int) sizeof(T), MAXCH);
+	constexpr int MINCH = (IsF16<T>::value ? FUSED : MAXCH == SMX_MAXCH) ? ATLEAST : 0;
 	using W = SmxWord<T>;
 	using WO = SmxWord<TO>;
 	static_assert(sizeof(T) == sizeof(TO), "in-register output packing needs equal widths");
@@ -389,22 +403,25 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 	};
 
 	/* chunks SMX_PF .. SMX_PF + RP - 1 of the next row are loaded a row ahead
-	 * into VGPRs; fp32 rows keep those registers for temporaries and load the
-	 * chunks past SMX_PF + RP at the top of their own row */
-	constexpr int RP = sizeof(T) < 4 ? SMX_MAXCH - SMX_PF : 0;
+	 * into VGPRs; fp32 rows keep those registers for temporaries, long rows
+	 * for their own chunks, and both load the chunks past SMX_PF + RP at the
+	 * top of their own row. (Loading them into their final registers during
+	 * the output pass, each after its predecessor's store, was slower: bf16
+	 * fused 4096 x 128256 383 -> 404 us, fp32 softmax 4096 x 65536 373 -> 386.) */
+	constexpr int RP = sizeof(T) < 4 && MAXCH == SMX_MAXCH ? SMX_MAXCH - SMX_PF : 0;
 	int row = blockIdx.x;
 	int par = 0;
-	R16 xr[SMX_MAXCH];
+	R16 xr[MAXCH];
 	R16 nx[RP > 0 ? RP : 1];
 	/* prologue: this workgroup's first row, LDS part and register part */
 	if (row < n_rows) {
 		const __amdgpu_buffer_rsrc_t r0 = make_rsrc(X + (long) row * n_cols, row_bytes);
 #pragma unroll
 		for (int c = 0; c < SMX_PF; c++)
-			if (c < nch) __builtin_amdgcn_raw_ptr_buffer_load_lds(r0, (lds_ptr_t) &pf[c * nt + wave_base], 16, voff, c * cstride, 0, BUF_AUX_NT);
+			if (c < MINCH || c < nch) __builtin_amdgcn_raw_ptr_buffer_load_lds(r0, (lds_ptr_t) &pf[c * nt + wave_base], 16, voff, c * cstride, 0, BUF_AUX_NT);
 #pragma unroll
 		for (int c = SMX_PF; c < SMX_PF + RP; c++)
-			if (c < nch) nx[c - SMX_PF] = buf_load16_nt(r0, voff, c * cstride);
+			if (c < MINCH || c < nch) nx[c - SMX_PF] = buf_load16_nt(r0, voff, c * cstride);
 		fetch_label(row);
 	}
 	WAIT_VMEM_ALL();
@@ -437,37 +454,41 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 		const uint32_t lab = FUSED ? labcell[wave] : 0xffffffffu;
 #pragma unroll
 		for (int c = 0; c < SMX_PF; c++)
-			if (c < nch) xr[c] = pf[c * nt + tid];
+			if (c < MINCH || c < nch) xr[c] = pf[c * nt + tid];
 		WAIT_LDS_ALL();
 #pragma unroll
 		for (int c = SMX_PF; c < SMX_PF + RP; c++)
-			if (c < nch) xr[c] = nx[c - SMX_PF];
-		if (RP < SMX_MAXCH - SMX_PF) {
+			if (c < MINCH || c < nch) xr[c] = nx[c - SMX_PF];
+		if (RP < MAXCH - SMX_PF) {
 			const __amdgpu_buffer_rsrc_t rin = make_rsrc(X + (long) row * n_cols, row_bytes);
 #pragma unroll
-			for (int c = SMX_PF + RP; c < SMX_MAXCH; c++)
-				if (c < nch) xr[c] = buf_load16_nt(rin, voff, c * cstride);
+			for (int c = SMX_PF + RP; c < MAXCH; c++)
+				if (c < MINCH || c < nch) xr[c] = buf_load16_nt(rin, voff, c * cstride);
 		}
 		/* the next row (requested during the max pass) and its label */
 		const bool has_next = next < n_rows;
 		const bool lab_ok = FUSED && lab < (uint32_t) n_cols;
 		const __amdgpu_buffer_rsrc_t rn = make_rsrc(X + (long) next * n_cols, has_next ? row_bytes : 0u);
 		auto issue_next = [&](int c) {
-			if (has_next && c < nch) {
+			if (has_next && (c < MINCH || c < nch)) {
 				if (c < SMX_PF) __builtin_amdgcn_raw_ptr_buffer_load_lds(rn, (lds_ptr_t) &pf[c * nt + wave_base], 16, voff, c * cstride, 0, BUF_AUX_NT);
 				else if (c < SMX_PF + RP) nx[c - SMX_PF] = buf_load16_nt(rn, voff, c * cstride);
 			}
 		};
 		if (has_next) fetch_label(next);
 
-		/* the last chunk's lanes past the row end (zeros from the range check)
-		 * become -inf, which leaves the max and both sums unchanged, so the
-		 * passes below need no per-lane mask */
+		/* the last chunk's lanes past the row end (zeros from the range
+		 * check) become -inf, which leaves the max and both sums unchanged,
+		 * so the passes need no per-lane mask: here, where the chunk has
+		 * landed, and with the chunk's use below for long rows, whose last
+		 * chunks are still on their way */
+		if (MAXCH == SMX_MAXCH) {
 #pragma unroll
-		for (int c = 0; c < SMX_MAXCH; c++) {
-			if (c == nch - 1 && c * nt + tid >= nv) {
+			for (int c = ATLEAST - 1; c < MAXCH; c++) {
+				if (c == nch - 1 && c * nt + tid >= nv) {
 #pragma unroll
-				for (int i = 0; i < 4; i++) xr[c].w[i] = W::NEG_INF;
+					for (int i = 0; i < 4; i++) xr[c].w[i] = W::NEG_INF;
+				}
 			}
 		}
 
@@ -499,10 +520,14 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 		 * has seen a finite value; mref64 = mref + 64, -inf until then */
 		float mref = 0.0f, mref64 = -__builtin_inff(), so = 0.0f;
 #pragma unroll
-		for (int c = 0; c < SMX_MAXCH; c++) {
+		for (int c = 0; c < MAXCH; c++) {
 			if (c >= SMX_PF) issue_next(c);
 			__builtin_amdgcn_sched_barrier(0);
-			if (c < nch) {
+			if (c < MINCH || c < nch) {
+				if (MAXCH > SMX_MAXCH && c >= ATLEAST - 1 && c == nch - 1 && c * nt + tid >= nv) {
+#pragma unroll
+					for (int i = 0; i < 4; i++) xr[c].w[i] = W::NEG_INF;
+				}
 				/* the chunk as floats (fp16: only where the label is read;
 				 * its max and terms come from the packed words) */
 				float f[VEC];
@@ -561,17 +586,17 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 		m = cells_max(m, mslots);
 		if (SX) so *= online_rescale(mref, m);   /* sx against the row max */
 #pragma unroll
-		for (int c = 0; c < SMX_MAXCH; c++) reg_barrier(xr[c]);
+		for (int c = 0; c < MAXCH; c++) reg_barrier(xr[c]);
 
 		/* sum pass: sd = sum exp(d) with d = rnd(x - m); the next row's LDS
 		 * part is requested here, chunk c before this row's chunk c (its
 		 * slots were emptied into xr at the top of this row) */
 		float sd0 = 0.0f, sd1 = 0.0f;
 #pragma unroll
-		for (int c = 0; c < SMX_MAXCH; c++) {
+		for (int c = 0; c < MAXCH; c++) {
 			if (c < SMX_PF) issue_next(c);
 			__builtin_amdgcn_sched_barrier(0);
-			if (c < nch) {
+			if (c < MINCH || c < nch) {
 				R16 o;
 #pragma unroll
 				for (int i = 0; i < 4; i++) {
@@ -594,8 +619,13 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 		const int next2 = __builtin_amdgcn_readfirstlane(nextcell[par]);
 		/* y = exp(d) / sd as one exp2: exp2(d * log2(e) - log2(sd)) */
 		const float nlog2s = -__builtin_amdgcn_logf(sd);
+		/* the differences are opaque again, so their unpacked floats are not
+		 * kept from the sum pass */
 #pragma unroll
-		for (int c = 0; c < SMX_MAXCH; c++) {
+		for (int c = 0; c < MINCH; c++) reg_barrier(xr[c]);
+#pragma unroll
+		for (int c = 0; c < MAXCH; c++) {
+			__builtin_amdgcn_sched_barrier(0);
 			/* every lane issues all SMX_MAXCH stores (chunks past the row lie
 			 * outside its buffer range and store nowhere), so the wait below
 			 * can count them */
@@ -632,8 +662,7 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 		 * stores drain behind it; waiting before the output pass instead held
 		 * the pass up until the LDS part requested during the sum pass had
 		 * arrived. */
-		static_assert(SMX_MAXCH == 16, "the wait below counts SMX_MAXCH stores");
-		__builtin_amdgcn_s_waitcnt(0x4F70);   /* vmcnt(16); expcnt, lgkmcnt at their maxima */
+		wait_vmem<MAXCH>();
 		if (FUSED && tid == 0 && loss) store_loss(loss, row, lab_ok ? fused_loss(sx, m, xlab_cell[par]) : __builtin_nanf(""));
 		par ^= 1;
 		row = next;
@@ -681,8 +710,8 @@ __device__ __forceinline__ void smx_stream(int n_rows, int n_cols, const T * X, 
 	}
 }
 
-/* Rows longer than the register path holds (more than SMX_MAXCH 16-byte
- * chunks per thread), 16-byte aligned: streaming passes over the row with
+/* Rows longer than the register paths hold (more than SMX_MAXCH 16-byte
+ * chunks per thread, SMX_LONG_MAXCH for 16-bit rows), 16-byte aligned: streaming passes over the row with
  * 16-byte accesses. The first pass finds the row max and, online, the sum of
  * exp(x - m) over the unrounded differences (each thread keeps its running
  * max and its sum against it, rescaled when the max grows; mref = 0 while the
@@ -706,9 +735,9 @@ __device__ __forceinline__ void smx_stream_vec(int n_rows, int n_cols, const T *
 	 * 879.6 -> 787.6 us, softmax 867.9 -> 750.3 us), 16-bit rows 8 chunks in
 	 * the softmax and 6 in the fused kernel, whose label and loss state leave
 	 * fewer registers (8 spilled there); held groups of two chunks, so the
-	 * first pass's working set stays small (4096 x 151936: bf16 fused 660.9
-	 * -> 591.1 us, softmax 651.1 -> 563.5 us, fp16 665.1 -> 588.5 and 654.3
-	 * -> 559.8 us). The outputs are bit-identical; the loss sum is rescaled
+	 * first pass's working set stays small (measured at 4096 x 151936, which
+	 * the 20-chunk register path holds now: bf16 fused 660.9 -> 591.1 us,
+	 * softmax 651.1 -> 563.5 us). The outputs are bit-identical; the loss sum is rescaled
 	 * at other chunks, so a loss can differ in its last bits. */
 	constexpr int HG = sizeof(T) == 4 ? 4 : (FUSED ? 3 : 4);
 	constexpr int UH = sizeof(T) == 4 ? U : 2;   /* chunks per held group */
@@ -877,7 +906,8 @@ template <typename T, typename TO, bool FUSED>
 __device__ __forceinline__ void smx(int n_rows, int n_cols, const T * X, TO * out, const uint32_t * labels, float * loss, float * mean_loss) {
 	constexpr int VEC = VecOf<T>::N;
 	const bool vec_ok = (n_cols % VEC == 0) && aligned16(X) && aligned16(out) && blockDim.x == SMX_THREADS
-						&& ((n_cols / VEC + SMX_THREADS - 1) / SMX_THREADS) <= SMX_MAXCH;
+						&& ((n_cols / VEC + SMX_THREADS - 1) / SMX_THREADS) <= SMX_MAXCH
+						&& ((n_cols / VEC + SMX_THREADS - 1) / SMX_THREADS) >= smx_regs_atleast((int) sizeof(T), SMX_MAXCH);
 	if (vec_ok) smx_regs<T, TO, FUSED>(n_rows, n_cols, X, out, labels, loss);
 	else if (sizeof(TO) == sizeof(T) && n_cols % VEC == 0 && aligned16(X) && aligned16(out) && blockDim.x == SMX_THREADS)
 		smx_stream_vec<T, FUSED>(n_rows, n_cols, X, reinterpret_cast<T *>(out), labels, loss);
@@ -904,6 +934,23 @@ __device__ __forceinline__ void smx(int n_rows, int n_cols, const T * X, TO * ou
 		*p = from_f<T>(to_f(*p) - 1.0f);                                                                               \
 	}
 
+/* 16-bit rows of 131,080 to 163,840 columns, held whole: 4096 x 151936 bf16
+ * fused 594 -> 461 us, softmax 557 -> 441 us (2.49 GB: 5.4 / 5.65 TB/s) against
+ * the streaming path, which reads most of such a row three times. Kernels of
+ * their own, so that 20 chunks do not cost the 16-chunk ones registers. */
+#define SMX_LONG_KERNELS(SUFFIX, PSUFFIX, T)                                                                             \
+	extern "C" __global__ void __launch_bounds__(SMX_THREADS) softmax_##PSUFFIX##_kernel_long_rows(int n_rows, int n_cols, \
+			T * X, T * out) {                                                                                          \
+		smx_regs<T, T, false, SMX_LONG_MAXCH>(n_rows, n_cols, X, out, nullptr, nullptr);                     \
+		smx_launch_end<false>(n_rows, nullptr, nullptr);                                                              \
+	}                                                                                                                  \
+	extern "C" __global__ void __launch_bounds__(SMX_THREADS) softmax_cross_entropy_loss_##SUFFIX##_kernel_long_rows(int n_rows, \
+			int n_cols, T * logits, uint32_t * labels, float * loss, float * mean_loss) {                              \
+		smx_regs<T, T, true, SMX_LONG_MAXCH>(n_rows, n_cols, logits, logits, labels, loss);                           \
+		smx_launch_end<true>(n_rows, loss, mean_loss);                                                                 \
+	}
+SMX_LONG_KERNELS(fp16, fp16_fp16, f16_t)
+SMX_LONG_KERNELS(bf16, bf16_bf16, bf16_t)
 SMX_KERNELS(fp32, fp32_fp32, float)
 SMX_KERNELS(fp16, fp16_fp16, f16_t)
 SMX_KERNELS(bf16, bf16_bf16, bf16_t)

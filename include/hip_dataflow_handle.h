@@ -78,8 +78,9 @@ typedef struct hip_launch_config {
  * by the launch configuration. */
 #define HIP_VARIANT_ROWS 1        /* "_rows" */
 #define HIP_VARIANT_WIDE_ROWS 2   /* "_wide_rows" */
-#define HIP_NUM_VARIANTS 2
-#define HIP_VARIANT_SUFFIXES {"_rows", "_wide_rows"}
+#define HIP_VARIANT_LONG_ROWS 3   /* "_long_rows" */
+#define HIP_NUM_VARIANTS 3
+#define HIP_VARIANT_SUFFIXES {"_rows", "_wide_rows", "_long_rows"}
 
 typedef struct hip_function Hip_Function;
 

@@ -734,7 +734,8 @@ def special_logits(dt, shape, seed):
 # half), short rows that share a workgroup, and more rows than one group of
 # the loss sum counts
 ROW_SHAPES = [(9, 2047, 0), (9, 2049, 1), (5, 4088, 0), (5, 4097, 3), (7, 16385, 0), (5, 32761, 1), (5, 32776, 0), (3, 65529, 5),
-              (3, 65544, 8), (2, 131001, 0), (2, 131073, 1), (259, 40001, 0), (2051, 200, 0), (523, 65, 7)]
+              (3, 65544, 8), (2, 131001, 0), (2, 131073, 1), (259, 40001, 0), (2051, 200, 0), (523, 65, 7),
+              (2, 163840, 0), (2, 163848, 0)]   # the last 16-bit row held in 20 chunks per thread, and one past it
 
 
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
