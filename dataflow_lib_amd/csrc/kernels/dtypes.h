@@ -16,6 +16,7 @@ struct f16_t { uint16_t bits; };
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_v;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_v;
 
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_v;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_v;
 
 /* one 16-byte memory vector */
@@ -246,6 +247,8 @@ __device__ __forceinline__ void vmem_wait_all() {
 __device__ __forceinline__ void reg_barrier(R16 & r) {
 	__asm__ volatile("" : "+v"(r.w[0]), "+v"(r.w[1]), "+v"(r.w[2]), "+v"(r.w[3]));
 }
+
+__device__ __forceinline__ void reg_barrier8(R8 & r) { __asm__ volatile("" : "+v"(r.w[0]), "+v"(r.w[1])); }
 
 /* A wave-uniform read of memory the kernel does not write, through the
  * scalar cache: an s_load (a read; nothing here stores through that cache),

@@ -19,8 +19,6 @@
 #include "reduce.h"
 #include "kernel_geometry.h"
 
-typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_v;
-
 __device__ __forceinline__ R8 ld8(const void * p) {
 	const u32x2_v v = __builtin_nontemporal_load(reinterpret_cast<const u32x2_v *>(p));
 	R8 r;
@@ -30,8 +28,6 @@ __device__ __forceinline__ R8 ld8(const void * p) {
 }
 
 __device__ __forceinline__ bool aligned8(const void * p) { return (((uintptr_t) p) & 7u) == 0; }
-
-__device__ __forceinline__ void reg_barrier8(R8 & r) { __asm__ volatile("" : "+v"(r.w[0]), "+v"(r.w[1])); }
 
 /* ---------------- RMSNorm backward: row slots ---------------- */
 
@@ -251,79 +247,6 @@ __device__ __forceinline__ void swiglu_bwd_fp8(long n, const TF * g, const TF * 
 
 /* ---------------- softmax ---------------- */
 
-/* Register rows: workgroups of F8_SMX_THREADS take rows block, block + grid,
- * ...; thread t holds the row's 8-byte pieces (8 fp8 values)
- * t + F8_SMX_THREADS j, j < F8_SMX_CH, so a row of up to
- * 8 * F8_SMX_CH * F8_SMX_THREADS columns is read from memory once, and each
- * wave's loads (8 bytes per lane) and stores (16 bytes per lane) cover
- * contiguous spans. Two workgroups share a CU, so one's loads overlap the
- * other's reductions and stores. Each pass decodes the pieces again (two
- * codes per instruction) instead of keeping the floats. */
-template <typename TF, typename TO>
-__device__ __forceinline__ void softmax_fp8_regs(int n_rows, int n_cols, const TF * X, TO * out, float * slots) {
-	const int np = n_cols / 8;
-	constexpr int nt = F8_SMX_THREADS;   /* the caller checked blockDim */
-	const int tid = (int) threadIdx.x;
-	const uint8_t * X8 = reinterpret_cast<const uint8_t *>(X);
-	/* rows through buffer ranges (the row is uniform over the workgroup):
-	 * 32-bit offsets, and pieces past the row load zero / store nowhere */
-	for (int row = blockIdx.x; row < n_rows; row += gridDim.x) {
-		R8 cur[F8_SMX_CH];
-		const __amdgpu_buffer_rsrc_t rx = make_rsrc(X8 + (long) row * n_cols, (uint32_t) n_cols);
-#pragma unroll
-		for (int j = 0; j < F8_SMX_CH; j++) {
-			if (nt * j < np) {
-				const u32x2_v v = __builtin_amdgcn_raw_buffer_load_b64(rx, (uint32_t) (tid + nt * j) * 8u, 0, BUF_AUX_NT);
-				cur[j].w[0] = v.x;
-				cur[j].w[1] = v.y;
-			}
-		}
-		float m = -__builtin_inff();
-#pragma unroll
-		for (int j = 0; j < F8_SMX_CH; j++) {
-			if (tid + nt * j < np) {
-				float f[8];
-				unpack8_fp8<TF>(cur[j], f);
-#pragma unroll
-				for (int e = 0; e < 8; e++) m = __builtin_elementwise_maximum(m, f[e]);
-			}
-		}
-		m = block_max(m, slots);
-		/* the pieces are opaque again after each pass, so the compiler
-		 * decodes them anew instead of keeping all 8 * F8_SMX_CH floats alive */
-#pragma unroll
-		for (int j = 0; j < F8_SMX_CH; j++) reg_barrier8(cur[j]);
-		float sd = 0.0f;
-#pragma unroll
-		for (int j = 0; j < F8_SMX_CH; j++) {
-			if (tid + nt * j < np) {
-				float f[8];
-				unpack8_fp8<TF>(cur[j], f);
-#pragma unroll
-				for (int e = 0; e < 8; e++) sd += exp_fast(rnd_in<TO>(f[e] - m));
-			}
-		}
-		float unused = 0.0f;
-		__syncthreads();   /* every wave has read the max cells */
-		block_sum2(sd, unused, slots);
-		const float nlog2s = -__builtin_amdgcn_logf(sd);
-#pragma unroll
-		for (int j = 0; j < F8_SMX_CH; j++) reg_barrier8(cur[j]);
-		const __amdgpu_buffer_rsrc_t ro = make_rsrc(out + (long) row * n_cols, (uint32_t) n_cols * 2u);
-#pragma unroll
-		for (int j = 0; j < F8_SMX_CH; j++) {
-			if (nt * j < np) {
-				float f[8];
-				unpack8_fp8<TF>(cur[j], f);
-#pragma unroll
-				for (int e = 0; e < 8; e++) f[e] = __builtin_amdgcn_exp2f(fmaf(rnd_in<TO>(f[e] - m), SMX_LOG2E, nlog2s));
-				buf_store16_nt(ro, (uint32_t) (tid + nt * j) * 16u, 0, pack16<TO>(f));
-			}
-		}
-		__syncthreads();   /* the cells are rewritten for the next row */
-	}
-}
-
 /* Long rows (f8_smx_pf_ok): one SMX_THREADS workgroup per CU; thread t holds
  * the row's 8-byte pieces t + SMX_THREADS j (j < F8_PF_PIECES) in registers
  * while the next row is requested, after this row's max reduction, so that
@@ -332,11 +255,9 @@ __device__ __forceinline__ void softmax_fp8_regs(int n_rows, int n_cols, const T
  * in the 8-byte layout, which takes other waves' loads, hence a barrier
  * after every wave has waited for its own), its second half into registers
  * (8-byte loads). The reductions' barriers wait for LDS only (cells_max /
- * cells_sum2), so the prefetch stays in flight across them. The LDS buffer is
- * 64 KB, so the two-workgroup register path of shorter rows, compiled into the
- * same kernel, still fits two workgroups per CU. Pieces past the row end load
- * zeros and are left out of the max and the sum; their stores fall outside
- * the row's range and store nothing. Rows are handed out as workgroups free
+ * cells_sum2), so the prefetch stays in flight across them. Pieces past the
+ * row end load zeros and are left out of the max and the sum; their stores
+ * fall outside the row's range and store nothing. Rows are handed out as workgroups free
  * up, as in the 16-bit softmax: each workgroup's first two rows are block and
  * block + grid, every later one a ticket of the code object's launch-wide row
  * counter (g_smx_sched), taken by thread 0 at the top of a row for the row
@@ -451,7 +372,7 @@ __device__ __forceinline__ void softmax_fp8_pf(int n_rows, int n_cols, const TF 
 	vmem_wait_all();
 }
 
-/* Other rows: three passes per row, the later ones re-reading the row (a
+/* Other rows (of more than 131,072 columns, or unaligned tensors): three passes per row, the later ones re-reading the row (a
  * row of fp8 is n_cols bytes, so they find it in cache): max, sum exp(d),
  * outputs. In both paths d = rnd_out(x - max), since the reference converts x
  * to the output type and subtracts there. */
@@ -461,10 +382,6 @@ __device__ __forceinline__ void softmax_fp8(int n_rows, int n_cols, const TF * X
 	if (blockDim.x == SMX_THREADS && f8_smx_pf_ok(n_cols) && aligned16(X) && aligned16(out)) {
 		softmax_fp8_pf<TF, TO>(n_rows, n_cols, X, out);
 		smx_launch_end<false>(n_rows, nullptr, nullptr);
-		return;
-	}
-	if (blockDim.x == F8_SMX_THREADS && f8_smx_regs_ok(n_cols) && aligned16(X) && aligned16(out)) {
-		softmax_fp8_regs<TF, TO>(n_rows, n_cols, X, out, slots);
 		return;
 	}
 	const bool vec = (n_cols % 8) == 0 && aligned8(X) && aligned16(out);

@@ -71,11 +71,6 @@
 #define F8_CPT 2
 #define F8_BWDX_WG_PER_CU 4
 
-/* fp8 -> 16-bit softmax (fp8_ops.hip): rows of up to 8 * F8_SMX_CH *
- * F8_SMX_THREADS columns held in registers, two workgroups per CU */
-#define F8_SMX_THREADS 512
-#define F8_SMX_CH 32
-
 /* embedding / copy_to_seq_context: one wave per row, 4 waves per workgroup */
 #define GS_WAVES 4
 
@@ -183,24 +178,32 @@ GEOM_FN int f8_smx_pf_ok(int n_cols) {
 	return n_cols >= F8_PF_MIN_COLS && (n_cols % 16) == 0 && n_cols / 8 <= F8_PF_PIECES * SMX_THREADS;
 }
 
-GEOM_FN int f8_smx_regs_ok(int n_cols) {
-	return n_cols > 0 && (n_cols % 8) == 0 && n_cols / 8 <= F8_SMX_CH * F8_SMX_THREADS;
-}
-
 /* softmax register-row paths: the fewest chunks per thread that a row there
  * has (smx_kernel_for sends shorter ones elsewhere) */
 GEOM_CONST int smx_regs_atleast(int elem_bytes, int maxch) {
 	return maxch > SMX_MAXCH ? SMX_MAXCH + 1 : (elem_bytes == 4 ? 6 : 8);
 }
 
-/* softmax "_rows" kernels: the 16-byte chunks a row's window can have
- * (SmxWindow), or 0 when input and output lie differently within a chunk */
+/* softmax "_rows" kernels: what a row's window (SmxWindow) starts on, less one:
+ * a 128-byte line, or 16 bytes where input and output lie differently within
+ * their lines and where the line's other elements would not fit beside the
+ * longest rows */
+GEOM_FN unsigned smx_rows_line(int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
+	if (elem_bytes == 1) return n_cols > 8 * 1024 * SMX_WIDE_ROWS_CH - 128 ? 15u : 127u;
+	return ((x ^ out) & 127ull) ? 15u : 127u;
+}
+
+/* The chunks (16 bytes, fp8 logits 8) a row's window can have, or 0 when input
+ * and output lie differently within a chunk (fp8 logits: are not both 16-byte
+ * aligned) */
 GEOM_FN int smx_rows_chunks(int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
 	const long bytes = (long) n_cols * elem_bytes;
-	const unsigned long long line = ((x ^ out) & 127ull) ? 15ull : 127ull;
-	if (((x ^ out) & 15ull) != 0ull || ((x | out) % (unsigned) elem_bytes) != 0ull) return 0;
-	const long slack = ((bytes & (long) line) | (long) (x & line)) ? (long) line : 0;
-	return (int) ((bytes + slack + 15) / 16);
+	const long chunk = elem_bytes == 1 ? 8 : 16;
+	const long line = (long) smx_rows_line(n_cols, elem_bytes, x, out);
+	if (elem_bytes == 1 ? ((x | out) & 15ull) != 0ull : ((x ^ out) & 15ull) != 0ull || ((x | out) % (unsigned) elem_bytes) != 0ull) return 0;
+	const long off = (bytes | (long) (x & 127ull)) & line;   /* rows start at multiples of its lowest bit */
+	const long slack = off == 0 ? 0 : (off % chunk == 0 ? line + 1 - chunk : line);
+	return (int) ((bytes + slack + chunk - 1) / chunk);
 }
 
 /* Waves per row for a kernel of ch chunks per thread, or 0 when 16 waves do
@@ -226,7 +229,11 @@ GEOM_FN int smx_rows_waves(int ch, int n_rows, int n_cols, int elem_bytes, unsig
  *   are many of them, go to the main kernel, which overlaps one row with the
  *   next on the same CU (1024 x 100000 bf16 78.5 us, wide 98.3; 4096 x 32000
  *   fp32 169.4, wide 184.1), unless they are unaligned, which it does not
- *   hold in registers (1024 x 128257 bf16 557 us, wide 116).
+ *   hold in registers (1024 x 128257 bf16 557 us, wide 116);
+ * - fp8 logits the same way: 12 waves of 8 chunks still share a CU with
+ *   another row (1024 x 48000 27.7 us, wide 30.3; 1024 x 50256 43.0, wide
+ *   31.6), and the main kernel overlaps rows from some 512 on (300 x 128256
+ *   41.4 us, wide 34.7; 1024 x 100000 68.4, wide 78.9).
  */
 #define SMX_MAIN 0
 #define SMX_ROWS 1
@@ -238,8 +245,12 @@ GEOM_FN int smx_kernel_for(int n_rows, int n_cols, int elem_bytes, unsigned long
 	const int few = n_rows <= SMX_FEW_ROWS;
 	/* the main kernel holds the row in registers too */
 	const int main_regs = ((x | out) & 15ull) == 0ull && ((long) n_cols * elem_bytes) % 16 == 0;
-	if (main_regs && elem_bytes < 4 && chunks > 1024 * SMX_MAXCH && ((long) n_cols * elem_bytes) / 16 <= 1024 * SMX_LONG_MAXCH) return SMX_LONG_ROWS;
+	if (main_regs && elem_bytes == 2 && chunks > 1024 * SMX_MAXCH && ((long) n_cols * elem_bytes) / 16 <= 1024 * SMX_LONG_MAXCH) return SMX_LONG_ROWS;
 	if (chunks == 0 || chunks > 1024 * SMX_WIDE_ROWS_CH) return SMX_MAIN;
+	if (elem_bytes == 1) {
+		if (chunks <= (few ? 1024 : 768) * SMX_ROWS_CH) return SMX_ROWS;
+		return (chunks <= 1024 * SMX_ROWS_CH || n_rows <= 2 * SMX_FEW_ROWS || !f8_smx_pf_ok(n_cols)) ? SMX_WIDE_ROWS : SMX_MAIN;
+	}
 	if (chunks <= 1024 * SMX_ROWS_CH && (few || chunks <= (elem_bytes < 4 ? 512 : 256) * SMX_ROWS_CH)) return SMX_ROWS;
 	if (!main_regs) return SMX_WIDE_ROWS;
 	if (elem_bytes == 4 && chunks > 6144 && n_rows >= 8 * SMX_FEW_ROWS) return SMX_MAIN;

@@ -1,6 +1,6 @@
 /*
- * Softmax and fused softmax + cross-entropy for rows of up to 131,072 16-bit
- * or 65,536 fp32 columns at any alignment: the "_rows" and "_wide_rows"
+ * Softmax and fused softmax + cross-entropy for rows of up to 131,072 fp8 or
+ * 16-bit or 65,536 fp32 columns at any alignment: the "_rows" and "_wide_rows"
  * kernels of softmax_xent.hip's ops (same arithmetic), chosen by
  * smx_kernel_for.
  *
@@ -15,14 +15,43 @@
  *    4096 x 32000  151 ->  92 us      187 ->  96 us  (524 MB: 5.7 / 5.5 TB/s)
  *    4096 x 50257  765 -> 156 us      687 -> 162 us  (823 MB: 5.3 / 5.1 TB/s)
  *    1024 x 128257 557 -> 116 us      588 -> 127 us
+ * and softmax of fp8 logits into bf16:
+ *    4096 x 1000    43 -> 6.3 us,  4096 x 32000 102 -> 71 us (393 MB: 5.5 TB/s),
+ *    1024 x 50257  171 -> 32 us,   1024 x 100001 373 -> 80 us
  */
 
-/* The 16-byte chunks that cover a row: the window starts at the 128-byte line
- * (16-byte chunk, where input and output lie differently within their lines)
- * that holds the row's first element, so that every wave's loads and stores
- * are whole lines however long the rows are. Elements [h, end) of the window
- * are the row's; the others belong to the neighbouring rows, are read with it
- * (a chunk never crosses a page) and never written. */
+/* A chunk: 16 bytes, or for fp8 logits, whose outputs are 16-bit, 8 bytes, so
+ * that a lane's output chunk is 16 bytes too. */
+template <typename T>
+struct SmxChunk {
+	static constexpr int N = VecOf<T>::N;
+	typedef R16 raw;
+	__device__ static __forceinline__ raw load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) { return buf_load16_nt(r, voff, soff); }
+	__device__ static __forceinline__ void unpack(const raw & r, float * f) { unpack16<T>(r, f); }
+};
+template <typename T>
+struct SmxChunkFp8 {
+	static constexpr int N = 8;
+	typedef R8 raw;
+	__device__ static __forceinline__ raw load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+		const u32x2_v v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, BUF_AUX_NT);
+		raw o;
+		o.w[0] = v.x;
+		o.w[1] = v.y;
+		return o;
+	}
+	__device__ static __forceinline__ void unpack(const raw & r, float * f) { unpack8_fp8<T>(r, f); }
+	__device__ static __forceinline__ void opaque(raw & r) { reg_barrier8(r); }
+};
+template <> struct SmxChunk<fp8e4m3_t> : SmxChunkFp8<fp8e4m3_t> {};
+template <> struct SmxChunk<fp8e5m2_t> : SmxChunkFp8<fp8e5m2_t> {};
+
+/* The chunks that cover a row: the window starts at the 128-byte line (16-byte
+ * chunk, where input and output lie differently within their lines) that
+ * holds the row's first element, so that every wave's loads and stores are
+ * whole lines however long the rows are. Elements [h, end) of the window are
+ * the row's; the others belong to the neighbouring rows, are read with it (a
+ * chunk never crosses a page) and never written. */
 struct SmxWindow {
 	const char * in;
 	char * out;
@@ -30,34 +59,20 @@ struct SmxWindow {
 	int chunks;
 };
 
-template <typename T>
-__device__ __forceinline__ SmxWindow smx_window(const T * X, T * out, int n_cols, int row) {
-	const uint64_t off = (uint64_t) row * (uint64_t) n_cols * sizeof(T);
-	const uint64_t a = (uint64_t) (uintptr_t) X + off, o = (uint64_t) (uintptr_t) out + off;
-	const uint64_t mask = ((a ^ o) & 127u) ? 15u : 127u;
+template <typename T, typename TO>
+__device__ __forceinline__ SmxWindow smx_window(const T * X, TO * out, int n_cols, int row) {
+	const int64_t first = (int64_t) row * n_cols;   /* the row's first element */
+	const uint64_t a = (uint64_t) (uintptr_t) (X + first);
+	/* outputs of another size: X and out are 16-byte aligned (smx_rows_chunks),
+	 * so the window's first element is a chunk's first in out too */
+	const uint64_t mask = smx_rows_line(n_cols, (int) sizeof(T), (unsigned long long) (uintptr_t) X, (unsigned long long) (uintptr_t) out);
 	SmxWindow w;
-	w.in = reinterpret_cast<const char *>(a & ~mask);
-	w.out = reinterpret_cast<char *>(o & ~mask);
 	w.h = (uint32_t) (a & mask) / (uint32_t) sizeof(T);
+	w.in = reinterpret_cast<const char *>(a & ~mask);
+	w.out = reinterpret_cast<char *>(out + (first - (int64_t) w.h));
 	w.end = w.h + (uint32_t) n_cols;
-	w.chunks = (int) ((w.end + VecOf<T>::N - 1) / VecOf<T>::N);
+	w.chunks = (int) ((w.end + SmxChunk<T>::N - 1) / SmxChunk<T>::N);
 	return w;
-}
-
-/* the window's elements outside the row become -inf */
-template <typename T>
-__device__ __forceinline__ void smx_mask_chunk(R16 & r, uint32_t pos, uint32_t h, uint32_t end) {
-	constexpr int PW = 4 / (int) sizeof(T);   /* elements per word */
-#pragma unroll
-	for (int i = 0; i < 4; i++) {
-		uint32_t keep = 0u;
-#pragma unroll
-		for (int e = 0; e < PW; e++) {
-			const uint32_t p = pos + (uint32_t) (i * PW + e);
-			if (p >= h && p < end) keep |= (PW == 1 ? 0xffffffffu : 0xffffu << (16 * e));
-		}
-		r.w[i] = (r.w[i] & keep) | (SmxWord<T>::NEG_INF & ~keep);
-	}
 }
 
 /* reductions over the `g` waves of a row, the waves' partials combined from
@@ -160,6 +175,32 @@ __device__ __forceinline__ void smx_rows_mean(const SmxGroup & g, unsigned arriv
 	if (lane == 0) *mean_loss = (float) (s / (double) n_rows);
 }
 
+/* the window's elements outside the row become -inf, in place (fp8, which has
+ * no infinity in E4M3, masks the unpacked values instead) */
+template <typename T>
+__device__ __forceinline__ void smx_mask_chunk(R16 & r, uint32_t pos, uint32_t h, uint32_t end) {
+	constexpr int PW = 4 / (int) sizeof(T);   /* elements per word */
+#pragma unroll
+	for (int i = 0; i < 4; i++) {
+		uint32_t keep = 0u;
+#pragma unroll
+		for (int e = 0; e < PW; e++) {
+			const uint32_t p = pos + (uint32_t) (i * PW + e);
+			if (p >= h && p < end) keep |= (PW == 1 ? 0xffffffffu : 0xffffu << (16 * e));
+		}
+		r.w[i] = (r.w[i] & keep) | (SmxWord<T>::NEG_INF & ~keep);
+	}
+}
+
+/* d = rnd(x - m) of a pair of fp8 values, in the 16-bit output type: opaque,
+ * so that both halves come from one packed convert */
+template <typename TO>
+__device__ __forceinline__ void smx_round2(const float * x_m, float * d) {
+	uint32_t w = SmxWord<TO>::pack(x_m);
+	__asm__ volatile("" : "+v"(w));
+	SmxWord<TO>::unpack(w, d);
+}
+
 /*
  * One row per `g` waves (smx_rows_waves: a wave alone, or a workgroup of g),
  * CH 16-byte chunks per thread, loaded at once, reduced twice and written;
@@ -171,11 +212,15 @@ __device__ __forceinline__ void smx_rows_mean(const SmxGroup & g, unsigned arriv
  * them by 1 / sum, one exponential less per element than forming them again
  * from the rounded differences, which the longest rows (CH = 16) do.
  */
-template <typename T, bool FUSED, int CH>
-__device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, T * out, const uint32_t * labels, float * loss, float * mean_loss) {
-	constexpr int VEC = VecOf<T>::N;
+template <typename T, typename TO, bool FUSED, int CH>
+__device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, TO * out, const uint32_t * labels, float * loss, float * mean_loss) {
+	using C = SmxChunk<T>;
+	constexpr int VEC = C::N;
+	constexpr int CB = VEC * (int) sizeof(T);   /* bytes of a chunk */
+	constexpr int OB = VEC * (int) sizeof(TO);
 	constexpr bool KEEP = CH * VEC <= 64;
-	using W = SmxWord<T>;
+	constexpr bool F8 = IsFp8<T>::value;
+	static_assert(OB == 16, "a chunk's outputs are one 16-byte store");
 	__shared__ float mcells[16];
 	__shared__ float scells[32];
 	__shared__ float xlab_cell[SMX_ROWS_PER_WG];
@@ -191,16 +236,16 @@ __device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, T 
 	const bool mean = FUSED && loss && mean_loss;
 	const int row = (g == 1) ? (int) blockIdx.x * SMX_ROWS_PER_WG + wv : (int) blockIdx.x;
 	if (row < n_rows) {   /* whole waves: no barrier where g == 1 */
-	const SmxWindow w = smx_window<T>(X, out, n_cols, row);
+	const SmxWindow w = smx_window<T, TO>(X, out, n_cols, row);
 	const int nch = (w.chunks + nt - 1) / nt;
-	const uint32_t voff = (uint32_t) t * 16u;
-	const __amdgpu_buffer_rsrc_t rin = make_rsrc(w.in, (uint32_t) w.chunks * 16u);
-	const __amdgpu_buffer_rsrc_t rout = make_rsrc(w.out, (uint32_t) w.chunks * 16u);
+	const uint32_t voff = (uint32_t) t * OB;
+	const __amdgpu_buffer_rsrc_t rin = make_rsrc(w.in, (uint32_t) w.chunks * CB);
+	const __amdgpu_buffer_rsrc_t rout = make_rsrc(w.out, (uint32_t) w.chunks * OB);
 
-	R16 x[CH];
+	typename C::raw x[CH];
 #pragma unroll
 	for (int c = 0; c < CH; c++)
-		if (c < nch) x[c] = buf_load16_nt(rin, voff, (uint32_t) (c * nt) * 16u);
+		if (c < nch) x[c] = C::load(rin, (uint32_t) t * CB, (uint32_t) (c * nt) * CB);
 	const uint32_t lab = FUSED ? load_scalar(labels + row) : 0xffffffffu;
 	const bool lab_ok = FUSED && lab < (uint32_t) n_cols;
 	/* the label's chunk, its thread and its element there */
@@ -209,19 +254,40 @@ __device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, T 
 	const int c_lab = lab_ok ? lab_chunk / nt : -1;
 	const int t_lab = lab_chunk - (lab_ok ? c_lab * nt : 0);
 	const int le = (int) (lab_pos % VEC);
-	/* only the first and the last chunk of a thread can hold elements
-	 * outside the row (h is below one line, 8 chunks) */
+	/* Elements outside the row are -inf, which changes neither the max nor
+	 * the sums. Only the first and the last chunk of a thread can hold any (h
+	 * is below one line). */
 	auto edge = [&](int c) { return c == 0 || c == nch - 1; };
+	auto partial = [&](int c) {
+		const uint32_t pos = (uint32_t) (c * nt + t) * VEC;
+		return pos < w.h || pos + VEC > w.end;
+	};
+	/* fp8: a chunk's values, unpacked anew in every pass */
+	auto values = [&](int c, float (&f)[VEC]) {
+		if constexpr (F8) C::opaque(x[c]);
+		C::unpack(x[c], f);
+		if (edge(c) && partial(c)) {
+			const uint32_t pos = (uint32_t) (c * nt + t) * VEC;
+#pragma unroll
+			for (int e = 0; e < VEC; e++)
+				if (pos + e < w.h || pos + e >= w.end) f[e] = -__builtin_inff();
+		}
+	};
 
 	float m = -__builtin_inff();
 #pragma unroll
 	for (int c = 0; c < CH; c++) {
 		if (c < nch) {
-			if (edge(c)) {
-				const uint32_t pos = (uint32_t) (c * nt + t) * VEC;
-				if (pos < w.h || pos + VEC > w.end) smx_mask_chunk<T>(x[c], pos, w.h, w.end);
+			if constexpr (F8) {
+				float f[VEC];
+				values(c, f);
+#pragma unroll
+				for (int e = 0; e < VEC; e++) m = __builtin_elementwise_maximum(m, f[e]);
 			}
-			m = chunk_max<T>(x[c], m);
+			else {
+				if (edge(c) && partial(c)) smx_mask_chunk<T>(x[c], (uint32_t) (c * nt + t) * VEC, w.h, w.end);
+				m = chunk_max<T>(x[c], m);
+			}
 		}
 	}
 	m = waves_max(m, mcells, g, wave, lane);
@@ -233,12 +299,26 @@ __device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, T 
 		if (c < nch) {
 			const bool lab_here = FUSED && c == c_lab && t == t_lab;
 			float x_m[VEC], d[VEC];
-			R16 o;
+			typename C::raw o;
+			if constexpr (F8) {
+				float f[VEC];
+				values(c, f);
 #pragma unroll
-			for (int i = 0; i < 4; i++) o.w[i] = W::diff(x[c].w[i], m, x_m + i * W::N, d + i * W::N);
+				for (int e = 0; e < VEC; e += 2) {
+					x_m[e] = f[e] - m;
+					x_m[e + 1] = f[e + 1] - m;
+					smx_round2<TO>(x_m + e, d + e);
+				}
+				o = x[c];
+			}
+			else {
+				using W = SmxWord<T>;
+#pragma unroll
+				for (int i = 0; i < 4; i++) o.w[i] = W::diff(x[c].w[i], m, x_m + i * W::N, d + i * W::N);
+			}
 			if (lab_here) {
 				float f[VEC];
-				unpack16<T>(x[c], f);
+				C::unpack(x[c], f);
 				float xl = f[0];
 #pragma unroll
 				for (int e = 1; e < VEC; e++)
@@ -268,7 +348,7 @@ __device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, T 
 #pragma unroll
 				for (int e = 0; e < VEC; e++) ef[c][e] = ev[e];
 			}
-			else x[c] = o;
+			else x[c] = o;   /* the differences, exact in T (fp8: the logits) */
 		}
 	}
 	float sd = sd0 + sd1;
@@ -290,30 +370,40 @@ __device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, T 
 				for (int e = 0; e < VEC; e++) f[e] = ef[c][e] * inv;
 			}
 			else {
-				unpack16<T>(x[c], f);
+				if constexpr (F8) {
+					C::opaque(x[c]);
+					C::unpack(x[c], f);
+#pragma unroll
+					for (int e = 0; e < VEC; e += 2) {
+						f[e] -= m;
+						f[e + 1] -= m;
+						smx_round2<TO>(f + e, f + e);
+					}
+				}
+				else C::unpack(x[c], f);
 #pragma unroll
 				for (int e = 0; e < VEC; e++) f[e] = __builtin_amdgcn_exp2f(fmaf(f[e], SMX_LOG2E, nlog2s));
 			}
-			R16 o = pack16<T>(f);
+			R16 o = pack16<TO>(f);
 			if (FUSED && c == c_lab && t == t_lab) {   /* rnd(y) - 1 */
-				unpack16<T>(o, f);
+				unpack16<TO>(o, f);
 #pragma unroll
 				for (int e = 0; e < VEC; e++)
 					if (e == le) f[e] -= 1.0f;
-				o = pack16<T>(f);
+				o = pack16<TO>(f);
 			}
 			if (edge(c)) {
 				const uint32_t pos = (uint32_t) (c * nt + t) * VEC;
-				if (pos >= w.h && pos + VEC <= w.end) buf_store16_nt(rout, voff, (uint32_t) (c * nt) * 16u, o);
+				if (pos >= w.h && pos + VEC <= w.end) buf_store16_nt(rout, voff, (uint32_t) (c * nt) * OB, o);
 				else {
-					T * p = reinterpret_cast<T *>(w.out);
-					unpack16<T>(o, f);
+					TO * p = reinterpret_cast<TO *>(w.out);
+					unpack16<TO>(o, f);
 #pragma unroll
 					for (int e = 0; e < VEC; e++)
-						if (pos + e >= w.h && pos + e < w.end) p[pos + e] = from_f<T>(f[e]);
+						if (pos + e >= w.h && pos + e < w.end) p[pos + e] = from_f<TO>(f[e]);
 				}
 			}
-			else buf_store16_nt(rout, voff, (uint32_t) (c * nt) * 16u, o);
+			else buf_store16_nt(rout, voff, (uint32_t) (c * nt) * OB, o);
 		}
 	}
 	}
@@ -329,11 +419,11 @@ __device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, T 
 #define SMX_ROWS_KERNEL(SUFFIX, PSUFFIX, T, VARIANT, CH)                                                               \
 	extern "C" __global__ void __launch_bounds__(SMX_THREADS) softmax_##PSUFFIX##_kernel_##VARIANT(int n_rows,         \
 			int n_cols, T * X, T * out) {                                                                              \
-		smx_rows<T, false, CH>(n_rows, n_cols, X, out, nullptr, nullptr, nullptr);                                     \
+		smx_rows<T, T, false, CH>(n_rows, n_cols, X, out, nullptr, nullptr, nullptr);                                     \
 	}                                                                                                                  \
 	extern "C" __global__ void __launch_bounds__(SMX_THREADS) softmax_cross_entropy_loss_##SUFFIX##_kernel_##VARIANT(  \
 			int n_rows, int n_cols, T * logits, uint32_t * labels, float * loss, float * mean_loss) {                  \
-		smx_rows<T, true, CH>(n_rows, n_cols, logits, logits, labels, loss, mean_loss);                                \
+		smx_rows<T, T, true, CH>(n_rows, n_cols, logits, logits, labels, loss, mean_loss);                                \
 	}
 #define SMX_ROWS_KERNELS(SUFFIX, PSUFFIX, T)                                                                           \
 	SMX_ROWS_KERNEL(SUFFIX, PSUFFIX, T, rows, SMX_ROWS_CH)                                                             \
@@ -342,3 +432,17 @@ __device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, T 
 SMX_ROWS_KERNELS(fp32, fp32_fp32, float)
 SMX_ROWS_KERNELS(fp16, fp16_fp16, f16_t)
 SMX_ROWS_KERNELS(bf16, bf16_bf16, bf16_t)
+
+#define SMX_FP8_ROWS_KERNEL(PSUFFIX, T, TO, VARIANT, CH)                                                               \
+	extern "C" __global__ void __launch_bounds__(SMX_THREADS) softmax_##PSUFFIX##_kernel_##VARIANT(int n_rows,         \
+			int n_cols, T * X, TO * out) {                                                                             \
+		smx_rows<T, TO, false, CH>(n_rows, n_cols, X, out, nullptr, nullptr, nullptr);                                 \
+	}
+#define SMX_FP8_ROWS_KERNELS(PSUFFIX, T, TO)                                                                           \
+	SMX_FP8_ROWS_KERNEL(PSUFFIX, T, TO, rows, SMX_ROWS_CH)                                                             \
+	SMX_FP8_ROWS_KERNEL(PSUFFIX, T, TO, wide_rows, SMX_WIDE_ROWS_CH)
+
+SMX_FP8_ROWS_KERNELS(fp8e4m3_fp16, fp8e4m3_t, f16_t)
+SMX_FP8_ROWS_KERNELS(fp8e4m3_bf16, fp8e4m3_t, bf16_t)
+SMX_FP8_ROWS_KERNELS(fp8e5m2_fp16, fp8e5m2_t, f16_t)
+SMX_FP8_ROWS_KERNELS(fp8e5m2_bf16, fp8e5m2_t, bf16_t)

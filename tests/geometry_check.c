@@ -1,0 +1,47 @@
+/* The launch rule of the softmax "_rows" kernels against what their rows
+ * really take, over storage types, lengths and places in memory: every row's
+ * window fits the chunks that smx_rows_chunks promised, the output window
+ * starts on a chunk, and the chosen kernel's waves hold the row. Prints what
+ * does not hold; the exit status is the number of such cases (at most 99). */
+#include <stdio.h>
+#include <stdint.h>
+
+#include "kernel_geometry.h"
+
+int main(void) {
+	static const unsigned long long offsets[] = {0, 16, 64, 112, 2, 6, 34, 128, 4, 12, 8, 1, 5};
+	static const int row_counts[] = {1, 200, 257, 5000};
+	const int n_off = (int) (sizeof(offsets) / sizeof(offsets[0]));
+	long bad = 0;
+	for (int e = 1; e <= 4; e *= 2) {
+		const int oe = e == 1 ? 2 : e;
+		const long chunk = e == 1 ? 8 : 16;
+		for (int i = 0; i < n_off * n_off; i++) {
+			const unsigned long long x = 4096 + offsets[i / n_off], o = 8192 + offsets[i % n_off];
+			if (x % e || o % oe) continue;
+			for (int n = 1; n < 140000; n += (n < 700 || (n > 130800 && n < 131200)) ? 1 : 1997) {
+				const int bound = smx_rows_chunks(n, e, x, o);
+				if (!bound) continue;
+				const unsigned line = smx_rows_line(n, e, x, o);
+				for (int r = 0; r < 130; r++) {
+					const unsigned long long a = x + (unsigned long long) r * n * e, h = a & line;
+					const long need = ((long) h + (long) n * e + chunk - 1) / chunk;
+					const unsigned long long out = o + (unsigned long long) r * n * oe - (h / e) * oe;
+					if (need > bound || (out & 15)) {
+						if (bad++ < 10) printf("elem %d, %d columns, x+%llu out+%llu, row %d: %ld chunks of %d, out %llu\n", e, n, x - 4096, o - 8192, r, need, bound, out & 15);
+					}
+				}
+				for (int k = 0; k < 4; k++) {
+					const int kernel = smx_kernel_for(row_counts[k], n, e, x, o);
+					if (kernel != SMX_ROWS && kernel != SMX_WIDE_ROWS) continue;
+					const int ch = kernel == SMX_ROWS ? SMX_ROWS_CH : SMX_WIDE_ROWS_CH;
+					const int g = smx_rows_waves(ch, row_counts[k], n, e, x, o);
+					if (g < 1 || g > 16 || (long) g * 64 * ch < bound) {
+						if (bad++ < 10) printf("elem %d, %d rows of %d columns: %d waves of %d chunks for %d\n", e, row_counts[k], n, g, ch, bound);
+					}
+				}
+			}
+		}
+	}
+	return bad > 99 ? 99 : (int) bad;
+}
