@@ -57,19 +57,22 @@ static int rms_check(const char * what, int n_rows, int n_cols, size_t elem) {
 	return 0;
 }
 
-/* workgroups of this function that are resident on the whole device at once;
- * the occupancy query is remembered per function for the last (block, LDS)
- * pair asked, so repeated submits of one shape do not repeat it */
-static long resident_groups(Dataflow_Handle * h, Hip_Function * f, int block, size_t lds) {
+/* workgroups of one of this function's kernels (0: the main one) that are
+ * resident on the whole device at once; the occupancy query is remembered per
+ * kernel for the last (block, LDS) pair asked, so repeated submits of one
+ * shape do not repeat it */
+static long resident_groups(Dataflow_Handle * h, Hip_Function * f, unsigned variant, int block, size_t lds) {
+	uint64_t * slot = &f->function_config.occupancy_memo[variant];
 	const uint64_t key = ((uint64_t) (unsigned) block << 40) | ((uint64_t) (lds & 0xffffffull) << 16);
-	const uint64_t memo = __atomic_load_n(&f->function_config.occupancy_memo, __ATOMIC_RELAXED);
+	const uint64_t memo = __atomic_load_n(slot, __ATOMIC_RELAXED);
 	int per_cu = 0;
 	if (memo != 0 && (memo & ~0xffffull) == key) {
 		per_cu = (int) (memo & 0xffffull);
 	}
 	else {
-		if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f->function_handle, block, lds) != hipSuccess || per_cu < 1) per_cu = 1;
-		if (lds <= 0xffffffull && per_cu <= 0xffff) __atomic_store_n(&f->function_config.occupancy_memo, key | (uint64_t) per_cu, __ATOMIC_RELAXED);
+		const hipFunction_t fn = variant == 0 ? f->function_handle : f->variant_handles[variant - 1];
+		if (!fn || hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, block, lds) != hipSuccess || per_cu < 1) per_cu = 1;
+		if (lds <= 0xffffffull && per_cu <= 0xffff) __atomic_store_n(slot, key | (uint64_t) per_cu, __ATOMIC_RELAXED);
 	}
 	return (long) per_cu * (long) dev(h)->cu_count;
 }
@@ -86,7 +89,7 @@ static void rms_rowwise(Hip_Launch_Config * c, Dataflow_Handle * h, Hip_Function
 	 * row in flight ahead, so it needs many rows per CU to hide latency */
 	const long groups_per_cu = (nv == 0) ? RMS_STREAM_GROUPS_PER_CU : MY_CEIL(rms_slots_per_cu(n_cols, (long) elem, arrays), (long) slots);
 	long grid = MY_MIN((long) MY_CEIL(n_rows, slots), (long) dev(h)->cu_count * groups_per_cu);
-	grid = MY_MIN(grid, resident_groups(h, f, (int) block, lds));
+	grid = MY_MIN(grid, resident_groups(h, f, 0, (int) block, lds));
 	set_1d(c, (unsigned) grid, block, lds);
 }
 
@@ -238,13 +241,26 @@ static int rope_config(Hip_Launch_Config * c, Dataflow_Handle * h, Hip_Function 
 	const size_t elem = arg_elem_bytes(f, 6);
 	const unsigned long long ptr_or = ptr_bits(ARG(op, 6, void *)) | ptr_bits(ARG(op, 7, void *));
 	uint64_t grid;
-	if (elem != 0 && rope_slot_ok(model_dim, num_kv_heads * head_dim, head_dim, (int) elem, ptr_or | extra_ptr_bits)) {
+	if (elem != 0 && rope_slot_ok(ROPE_SLOT_THREADS, model_dim, num_kv_heads * head_dim, head_dim, (int) elem, ptr_or | extra_ptr_bits)) {
 		/* vector path: one workgroup per token at a time, persistent, as many
 		 * per CU as the kernel's registers allow (at most ROPE_SLOT_WG_PER_CU) */
-		grid = MY_MIN((uint64_t) dev(h)->cu_count * ROPE_SLOT_WG_PER_CU, (uint64_t) resident_groups(h, f, ROPE_SLOT_THREADS, 0));
-		const uint64_t tg = (uint64_t) rope_tokens_per_group(model_dim, num_kv_heads * head_dim, (int) elem);
+		uint64_t tg = (uint64_t) rope_tokens_per_group((long) n_tokens, model_dim, num_kv_heads * head_dim, (int) elem);
+		const unsigned variant = tg > 1 ? HIP_VARIANT_MULTI : 0;
+		if (variant == 0 && elem == 1 && rope_fp8_pairs(model_dim, num_kv_heads * head_dim)) tg = 2;
+		grid = MY_MIN((uint64_t) dev(h)->cu_count * ROPE_SLOT_WG_PER_CU,
+					  (uint64_t) resident_groups(h, f, variant, ROPE_SLOT_THREADS, 0));
 		grid = MY_MIN(MY_CEIL(n_tokens, tg), grid);
 		set_1d(c, (unsigned) grid, ROPE_SLOT_THREADS, 0);
+		c->variant = variant;
+		return 0;
+	}
+	/* rows of more chunks than that, but not than twice that: workgroups of
+	 * ROPE_WIDE_THREADS */
+	if (elem > 1 && rope_slot_ok(ROPE_WIDE_THREADS, model_dim, num_kv_heads * head_dim, head_dim, (int) elem, ptr_or | extra_ptr_bits)) {
+		grid = MY_MIN((uint64_t) dev(h)->cu_count * ROPE_WIDE_WG_PER_CU,
+					  (uint64_t) resident_groups(h, f, HIP_VARIANT_WIDE_ROWS, ROPE_WIDE_THREADS, 0));
+		set_1d(c, (unsigned) MY_MIN(n_tokens, grid), ROPE_WIDE_THREADS, 0);
+		c->variant = HIP_VARIANT_WIDE_ROWS;
 		return 0;
 	}
 	/* element path: one wave per token, looping; four workgroups per CU */

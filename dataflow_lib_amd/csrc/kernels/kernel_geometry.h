@@ -61,6 +61,8 @@
  * four, the fused KV-cache variant's three, and the launch takes the smaller
  * of this and what the kernel's registers leave resident */
 #define ROPE_SLOT_WG_PER_CU 4
+#define ROPE_WIDE_THREADS 512
+#define ROPE_WIDE_WG_PER_CU 2
 
 /* fp8 x 16-bit RMSNorm backward (fp8_ops.hip): rows in 8-element chunks
  * (8 bytes of each fp8 operand, 16 of each 16-bit one); a row slot of TPR
@@ -257,20 +259,39 @@ GEOM_FN int smx_kernel_for(int n_rows, int n_cols, int elem_bytes, unsigned long
 	return chunks <= 1024 * SMX_ROWS_CH ? SMX_WIDE_ROWS : SMX_MAIN;
 }
 
-/* RoPE vector path: tokens per workgroup step. fp8 rows are half as long as
- * bf16 ones, so two tokens go together when their Q and K chunks fit the
- * slot's registers. */
-#define ROPE_TG2_QJ 2   /* Q chunks per thread in a two-token step */
-GEOM_FN int rope_tokens_per_group(int model_dim, int kv_dim, int elem_bytes) {
-	if (elem_bytes != 1) return 1;
-	return (2 * (model_dim / 16) <= ROPE_SLOT_THREADS * ROPE_TG2_QJ && 2 * (kv_dim / 16) <= ROPE_SLOT_THREADS * ROPE_KJ) ? 2 : 1;
+/* RoPE vector path: fp8 rows are half as long as bf16 ones, so the main kernel
+ * takes two tokens at a time when their Q and K chunks fit its registers. */
+#define ROPE_TG_QJ 2   /* Q chunks per thread in a step of several tokens */
+GEOM_FN int rope_fp8_pairs(int model_dim, int kv_dim) {
+	return 2 * (model_dim / 16) <= ROPE_SLOT_THREADS * ROPE_TG_QJ && 2 * (kv_dim / 16) <= ROPE_SLOT_THREADS * ROPE_KJ;
 }
 
-/* RoPE: whether the vector (slot) path applies */
-GEOM_FN int rope_slot_ok(int model_dim, int kv_dim, int head_dim, int elem_bytes, unsigned long long ptr_or) {
+/* Tokens per step of the "_multi" kernels, or 1 where the main kernel runs:
+ * four, else two, that fit ROPE_TG_QJ Q chunks per thread, from a step per CU
+ * on; else two of ROPE_QJ. A step's fp64 sin/cos tables take a wave about a
+ * microsecond, which rows of 1-2 KB do not hide: 8192 x (16 + 4) x 64 bf16 15.0
+ * -> 8.9 us with four (42 MB: 4.7 TB/s), 16384 x (8 + 8) x 64 26.2 -> 13.5,
+ * with the KV cache 22.2 -> 12.9 and 43.7 -> 21.8; two tokens of 8 KB rows gain
+ * once every CU has several steps (x (32 + 8) x 128, main -> two: 1024 tokens
+ * 5.4 -> 5.5 us, 1531 7.4 -> 6.6, 2048 9.4 -> 8.6, 8192 29.6 -> 29.2, with the
+ * KV cache 7.1 -> 7.5, 9.4 -> 8.9, 12.3 -> 10.8, 37.8 -> 36.1). fp8 takes two
+ * in its main kernel already. */
+GEOM_FN int rope_tokens_per_group(long n_tokens, int model_dim, int kv_dim, int elem_bytes) {
+	const int nvq = model_dim * elem_bytes / 16, nvk = kv_dim * elem_bytes / 16;
+	int tg = 4;
+	for (; tg > 1; tg /= 2) {
+		if (tg * nvq <= ROPE_SLOT_THREADS * ROPE_TG_QJ && tg * nvk <= ROPE_SLOT_THREADS * ROPE_KJ && n_tokens >= tg * 256L) break;
+	}
+	if (elem_bytes == 1) return tg == 4 ? 4 : 1;
+	if (tg == 1 && 2 * nvq <= ROPE_SLOT_THREADS * ROPE_QJ && 2 * nvk <= ROPE_SLOT_THREADS * ROPE_KJ && n_tokens >= 1280) return 2;
+	return tg;
+}
+
+/* RoPE: whether the vector (slot) path applies with workgroups of `threads` */
+GEOM_FN int rope_slot_ok(int threads, int model_dim, int kv_dim, int head_dim, int elem_bytes, unsigned long long ptr_or) {
 	const int vec = 16 / elem_bytes;
 	if ((head_dim % vec) != 0 || (ptr_or & 15ull) != 0ull) return 0;
-	return (model_dim / vec) <= ROPE_SLOT_THREADS * ROPE_QJ && (kv_dim / vec) <= ROPE_SLOT_THREADS * ROPE_KJ;
+	return (model_dim / vec) <= threads * ROPE_QJ && (kv_dim / vec) <= threads * ROPE_KJ;
 }
 
 #endif

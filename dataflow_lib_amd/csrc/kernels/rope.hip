@@ -196,12 +196,11 @@ __device__ __forceinline__ int rope_pair_of(int chunk, int head_dim, bool pow2) 
  * 0..TG-1 build its tokens' cos/sin tables into the other half of a
  * double-buffered LDS table, while this group is rotated and stored; one
  * barrier per group. */
-template <typename T, bool BWD, bool KV = false, int TG = 1, int QJ = ROPE_QJ>
+template <typename T, bool BWD, bool KV = false, int TG = 1, int QJ = ROPE_QJ, int NT = ROPE_SLOT_THREADS>
 __device__ __forceinline__ void rope_slot(long n_tokens, int model_dim, int head_dim, int kv_dim, int theta,
 											const int * seq_positions, T * X_q, T * X_k, KvCache<T> kv = KvCache<T>{}) {
-	static_assert(!KV || TG == 1, "the KV-cache scatter runs one token per step");
 	constexpr int VEC = VecOf<T>::N;
-	constexpr int NT = ROPE_SLOT_THREADS;
+	static_assert(TG <= NT / 64, "a wave per token's table");
 	__shared__ float ang[ROPE_MAX_HEAD_DIM / 2];
 	__shared__ __attribute__((aligned(16))) float2 tab[2][TG][ROPE_MAX_HEAD_DIM / 2];
 	const int tid = threadIdx.x;
@@ -218,6 +217,10 @@ __device__ __forceinline__ void rope_slot(long n_tokens, int model_dim, int head
 	 * of the chunk's token in the group (one index per chunk) */
 	constexpr int TS = ROPE_MAX_HEAD_DIM / 2;
 	int iq[QJ], ik[ROPE_KJ];
+	/* fused KV-cache scatter with several tokens per step: the context rows
+	 * of the step's tokens, and of each owned K chunk its token and byte */
+	__shared__ T * ctx_rows[2][KV && TG > 1 ? TG : 1][2];
+	int tk[KV && TG > 1 ? ROPE_KJ : 1];
 #pragma unroll
 	for (int j = 0; j < QJ; j++) {
 		const int c = tid + NT * j;
@@ -229,6 +232,7 @@ __device__ __forceinline__ void rope_slot(long n_tokens, int model_dim, int head
 		const int c = tid + NT * j;
 		const int tg = (TG == 1 || nvk == 0) ? 0 : c / nvk;
 		ik[j] = (tg < TG ? tg : 0) * TS + rope_pair_of<T>(c, head_dim, pow2);
+		if (KV && TG > 1) tk[j] = tg;
 	}
 
 	/* the cos/sin tables of group g's tokens into tab[b] (wave i builds token i) */
@@ -236,6 +240,14 @@ __device__ __forceinline__ void rope_slot(long n_tokens, int model_dim, int head
 		const long t = g * TG + wv;
 		if (wv >= TG || t >= n_tokens) return;
 		const float fpos = (float) load_scalar(seq_positions + t);
+		if (KV && TG > 1 && kv_dim > 0) {
+			T * kr = kv.row(t, kv_dim, seq_positions, false);
+			T * vr = kv.row(t, kv_dim, seq_positions, true);
+			if (lane == 0) {
+				ctx_rows[b][wv][0] = kr;
+				ctx_rows[b][wv][1] = vr;
+			}
+		}
 		for (int p = lane; p < half; p += 64) {
 			const float arg = fpos * ang[p];
 			double sd, cd;
@@ -260,10 +272,10 @@ __device__ __forceinline__ void rope_slot(long n_tokens, int model_dim, int head
 		for (int j = 0; j < ROPE_KJ; j++)
 			if (NT * j < TG * nvk) k[j] = buf_load16_nt(rk, (uint32_t) (tid + NT * j) * 16u, 0);
 		if (KV) {
-			const __amdgpu_buffer_rsrc_t rv = make_rsrc(kv.values + t * kv_dim, kbytes);
+			const __amdgpu_buffer_rsrc_t rv = make_rsrc(kv.values + t * kv_dim, span(g, kbytes));
 #pragma unroll
 			for (int j = 0; j < VJ; j++)
-				if (NT * j < nvk) v[j] = buf_load16_nt(rv, (uint32_t) (tid + NT * j) * 16u, 0);
+				if (NT * j < TG * nvk) v[j] = buf_load16_nt(rv, (uint32_t) (tid + NT * j) * 16u, 0);
 		}
 	};
 	/* fp8 outputs keep 3 (E4M3) or 2 (E5M2) mantissa bits, so they take the
@@ -319,7 +331,7 @@ __device__ __forceinline__ void rope_slot(long n_tokens, int model_dim, int head
 		/* fused KV-cache scatter: this token's context rows (scalar reads) */
 		T * kctx = nullptr;
 		T * vctx = nullptr;
-		if (KV && kv_dim > 0) {
+		if (KV && TG == 1 && kv_dim > 0) {
 			kctx = kv.row(t, kv_dim, seq_positions, false);
 			vctx = kv.row(t, kv_dim, seq_positions, true);
 		}
@@ -339,7 +351,33 @@ __device__ __forceinline__ void rope_slot(long n_tokens, int model_dim, int head
 				buf_store16_aux<BUF_AUX_DEV | BUF_AUX_NT>(rk, (uint32_t) (tid + NT * j) * 16u, 0, k[j]);
 			}
 		}
-		if (KV && kv_dim > 0) {
+		if (KV && TG > 1) {
+			/* each chunk to its own token's context rows (one at a time,
+			 * so the tokens need not lie in one context) */
+#pragma unroll
+			for (int j = 0; j < ROPE_KJ; j++) {
+				const int c = tid + NT * j;
+				if (NT * j < TG * nvk && tk[j] < TG && t * TG + tk[j] < n_tokens && c < TG * nvk) {
+					const int cc = c - tk[j] * nvk;
+					T * kr = ctx_rows[b][tk[j]][0] + cc * VEC;
+					T * vr = ctx_rows[b][tk[j]][1] + cc * VEC;
+					if (aligned16(kr) && aligned16(vr)) {
+						*reinterpret_cast<R16 *>(kr) = k[j];
+						*reinterpret_cast<R16 *>(vr) = v[j];
+					}
+					else {
+						const T * ke = reinterpret_cast<const T *>(&k[j]);
+						const T * ve = reinterpret_cast<const T *>(&v[j]);
+#pragma unroll
+						for (int e = 0; e < VEC; e++) {
+							kr[e] = ke[e];
+							vr[e] = ve[e];
+						}
+					}
+				}
+			}
+		}
+		else if (KV && kv_dim > 0) {
 			/* context rows are 16-byte aligned unless the caller's contexts
 			 * are not (a workgroup-uniform test per token); they are stored
 			 * with the default cache policy (config-3 shapes: 40.8 -> 38.0 us
@@ -391,11 +429,11 @@ __device__ __forceinline__ void rope_dispatch(uint64_t N, int model_dim, int hea
 	const int kv_dim = num_kv_heads * head_dim;
 	unsigned long long ptr_or = (unsigned long long) (uintptr_t) X_q | (unsigned long long) (uintptr_t) X_k;
 	if (KV) ptr_or |= (unsigned long long) (uintptr_t) kv.values;
-	if (blockDim.x == ROPE_SLOT_THREADS && rope_slot_ok(model_dim, kv_dim, head_dim, (int) sizeof(T), ptr_or)) {
+	if (blockDim.x == ROPE_SLOT_THREADS && rope_slot_ok(ROPE_SLOT_THREADS, model_dim, kv_dim, head_dim, (int) sizeof(T), ptr_or)) {
 		const long n_tokens = (long) (N / (uint64_t) model_dim);
 		if constexpr (!KV && IsFp8<T>::value) {
-			if (rope_tokens_per_group(model_dim, kv_dim, (int) sizeof(T)) == 2) {
-				rope_slot<T, BWD, false, 2, ROPE_TG2_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k);
+			if (rope_fp8_pairs(model_dim, kv_dim)) {
+				rope_slot<T, BWD, false, 2, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k);
 				return;
 			}
 		}
@@ -405,25 +443,59 @@ __device__ __forceinline__ void rope_dispatch(uint64_t N, int model_dim, int hea
 		rope_impl<T, BWD, KV>(N, model_dim, head_dim, num_kv_heads, theta, seq_positions, X_q, X_k, kv);
 }
 
-#define ROPE_KERNELS(SUFFIX, T)                                                                                     \
-	extern "C" __global__ void __launch_bounds__(256) rope_##SUFFIX##_kernel(uint64_t N, int model_dim, int head_dim, \
-			int num_kv_heads, int theta, int * seq_positions, T * X_q, T * X_k) {                                    \
-		rope_dispatch<T, false>(N, model_dim, head_dim, num_kv_heads, theta, seq_positions, X_q, X_k);              \
-	}                                                                                                               \
-	extern "C" __global__ void __launch_bounds__(256) rope_bwd_x_##SUFFIX##_kernel(uint64_t N, int model_dim, int head_dim, \
-			int num_kv_heads, int theta, int * seq_positions, T * dX_q, T * dX_k) {                                  \
-		rope_dispatch<T, true>(N, model_dim, head_dim, num_kv_heads, theta, seq_positions, dX_q, dX_k);             \
+/* the "_multi" kernels: several tokens per step (rope_tokens_per_group) */
+template <typename T, bool BWD, bool KV = false>
+__device__ __forceinline__ void rope_multi(uint64_t N, int model_dim, int head_dim, int num_kv_heads, int theta,
+											const int * seq_positions, T * X_q, T * X_k, KvCache<T> kv = KvCache<T>{}) {
+	const int kv_dim = num_kv_heads * head_dim;
+	const long n_tokens = (long) (N / (uint64_t) model_dim);
+	if constexpr (!IsFp8<T>::value) {
+		if (2 * (model_dim / VecOf<T>::N) > ROPE_SLOT_THREADS * ROPE_TG_QJ) {
+			rope_slot<T, BWD, KV, 2, ROPE_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
+			return;
+		}
 	}
+	if (rope_tokens_per_group(n_tokens, model_dim, kv_dim, (int) sizeof(T)) == 4)
+		rope_slot<T, BWD, KV, 4, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
+	else
+		rope_slot<T, BWD, KV, 2, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
+}
+
+#define ROPE_KERNELS(SUFFIX, T)                                                                                     \
+	ROPE_KERNEL(SUFFIX, T, kernel, rope_dispatch, ROPE_SLOT_THREADS)                                                \
+	ROPE_KERNEL(SUFFIX, T, kernel_multi, rope_multi, ROPE_SLOT_THREADS)                                             \
+	ROPE_KERNEL(SUFFIX, T, kernel_wide_rows, rope_wide, ROPE_WIDE_THREADS)
+#define ROPE_KERNEL(SUFFIX, T, NAME, IMPL, NT)                                                                        \
+	extern "C" __global__ void __launch_bounds__(NT) rope_##SUFFIX##_##NAME(uint64_t N, int model_dim, int head_dim, \
+			int num_kv_heads, int theta, int * seq_positions, T * X_q, T * X_k) {                                    \
+		IMPL<T, false>(N, model_dim, head_dim, num_kv_heads, theta, seq_positions, X_q, X_k);                       \
+	}                                                                                                               \
+	extern "C" __global__ void __launch_bounds__(NT) rope_bwd_x_##SUFFIX##_##NAME(uint64_t N, int model_dim, int head_dim, \
+			int num_kv_heads, int theta, int * seq_positions, T * dX_q, T * dX_k) {                                  \
+		IMPL<T, true>(N, model_dim, head_dim, num_kv_heads, theta, seq_positions, dX_q, dX_k);             \
+	}
+
+/* the "_wide_rows" kernels: rows past ROPE_SLOT_THREADS threads' chunks */
+template <typename T, bool BWD, bool KV = false>
+__device__ __forceinline__ void rope_wide(uint64_t N, int model_dim, int head_dim, int num_kv_heads, int theta,
+											const int * seq_positions, T * X_q, T * X_k, KvCache<T> kv = KvCache<T>{}) {
+	rope_slot<T, BWD, KV, 1, ROPE_QJ, ROPE_WIDE_THREADS>((long) (N / (uint64_t) model_dim), model_dim, head_dim, num_kv_heads * head_dim,
+														theta, seq_positions, X_q, X_k, kv);
+}
 
 /* RoPE fused with the KV-cache scatter (no reference counterpart; the
  * reference notes the fusion at attention/rope.cu:50-54): rope forward on Q
  * and K in place, and the rotated K row and the V row of token t written to
  * rows p and S + p of its context, as copy_to_seq_context does. */
 #define ROPE_KV_KERNELS(SUFFIX, T)                                                                                  \
-	extern "C" __global__ void __launch_bounds__(256) rope_copy_to_seq_context_##SUFFIX##_kernel(uint64_t N,       \
+	ROPE_KV_KERNEL(SUFFIX, T, kernel, rope_dispatch, ROPE_SLOT_THREADS)                                             \
+	ROPE_KV_KERNEL(SUFFIX, T, kernel_multi, rope_multi, ROPE_SLOT_THREADS)                                          \
+	ROPE_KV_KERNEL(SUFFIX, T, kernel_wide_rows, rope_wide, ROPE_WIDE_THREADS)
+#define ROPE_KV_KERNEL(SUFFIX, T, NAME, IMPL, NT)                                                                     \
+	extern "C" __global__ void __launch_bounds__(NT) rope_copy_to_seq_context_##SUFFIX##_##NAME(uint64_t N,       \
 			int model_dim, int head_dim, int num_kv_heads, int theta, int * seq_positions, T * X_q, T * X_k,         \
 			T * values, uint64_t * seq_context_ptrs, int * seq_context_sizes) {                                      \
-		rope_dispatch<T, false, true>(N, model_dim, head_dim, num_kv_heads, theta, seq_positions, X_q, X_k,         \
+		IMPL<T, false, true>(N, model_dim, head_dim, num_kv_heads, theta, seq_positions, X_q, X_k,         \
 									  KvCache<T>{values, seq_context_ptrs, seq_context_sizes});                      \
 	}
 
@@ -435,11 +507,13 @@ ROPE_KV_KERNELS(fp16, f16_t)
 ROPE_KV_KERNELS(bf16, bf16_t)
 
 /* fp8 forward only (reference: rope.cu:183-300; rope_bwd_x has no fp8 kernels) */
-#define ROPE_FP8_KERNEL(SUFFIX, T)                                                                                  \
-	extern "C" __global__ void __launch_bounds__(256, ROPE_SLOT_WG_PER_CU) rope_##SUFFIX##_kernel(uint64_t N, int model_dim, int head_dim, \
+#define ROPE_FP8_KERNEL(SUFFIX, T, NAME, IMPL)                                                                      \
+	extern "C" __global__ void __launch_bounds__(256, ROPE_SLOT_WG_PER_CU) rope_##SUFFIX##_##NAME(uint64_t N, int model_dim, int head_dim, \
 			int num_kv_heads, int theta, int * seq_positions, T * X_q, T * X_k) {                                    \
-		rope_dispatch<T, false>(N, model_dim, head_dim, num_kv_heads, theta, seq_positions, X_q, X_k);              \
+		IMPL<T, false>(N, model_dim, head_dim, num_kv_heads, theta, seq_positions, X_q, X_k);                       \
 	}
 
-ROPE_FP8_KERNEL(fp8e4m3, fp8e4m3_t)
-ROPE_FP8_KERNEL(fp8e5m2, fp8e5m2_t)
+ROPE_FP8_KERNEL(fp8e4m3, fp8e4m3_t, kernel, rope_dispatch)
+ROPE_FP8_KERNEL(fp8e4m3, fp8e4m3_t, kernel_multi, rope_multi)
+ROPE_FP8_KERNEL(fp8e5m2, fp8e5m2_t, kernel, rope_dispatch)
+ROPE_FP8_KERNEL(fp8e5m2, fp8e5m2_t, kernel_multi, rope_multi)

@@ -47,6 +47,16 @@ typedef struct hip_device_info {
 	char arch_name[64];
 } Hip_Device_Info;
 
+/* Further kernels of an op, with the same parameters, for shapes that its main
+ * kernel is not the best for: "<symbol>" + suffix in the code object, chosen
+ * by the launch configuration. */
+#define HIP_VARIANT_ROWS 1        /* "_rows" */
+#define HIP_VARIANT_WIDE_ROWS 2   /* "_wide_rows" */
+#define HIP_VARIANT_LONG_ROWS 3   /* "_long_rows" */
+#define HIP_VARIANT_MULTI 4       /* "_multi" */
+#define HIP_NUM_VARIANTS 4
+#define HIP_VARIANT_SUFFIXES {"_rows", "_wide_rows", "_long_rows", "_multi"}
+
 typedef struct hip_function_config {
 	int func_max_smem;
 	int func_max_threads_per_block;
@@ -54,10 +64,11 @@ typedef struct hip_function_config {
 	 * per-launch partial results in the code object's module-scope scratch:
 	 * the handle orders such functions across its streams (Hip_Context) */
 	int shares_module_scratch;
-	/* last occupancy query of the launch-config library, packed as
+	/* per kernel (0 the main one, then the variants) the last occupancy
+	 * query of the launch-config library, packed as
 	 * block << 40 | LDS bytes << 16 | workgroups per CU (0: none yet); read and
 	 * written as one 64-bit word, so concurrent submits see a whole entry */
-	uint64_t occupancy_memo;
+	uint64_t occupancy_memo[HIP_NUM_VARIANTS + 1];
 } Hip_Function_Config;
 
 typedef struct hip_launch_config {
@@ -72,15 +83,6 @@ typedef struct hip_launch_config {
 	 * variant_handles[i - 1] */
 	unsigned int variant;
 } Hip_Launch_Config;
-
-/* Further kernels of an op, with the same parameters, for shapes that its main
- * kernel is not the best for: "<symbol>" + suffix in the code object, chosen
- * by the launch configuration. */
-#define HIP_VARIANT_ROWS 1        /* "_rows" */
-#define HIP_VARIANT_WIDE_ROWS 2   /* "_wide_rows" */
-#define HIP_VARIANT_LONG_ROWS 3   /* "_long_rows" */
-#define HIP_NUM_VARIANTS 3
-#define HIP_VARIANT_SUFFIXES {"_rows", "_wide_rows", "_long_rows"}
 
 typedef struct hip_function Hip_Function;
 

@@ -209,6 +209,7 @@ def test_rms_norm_bwd_w_fp8_too_wide_is_refused(hdl):
 ROPE_CASES = [(8192, 32, 8, 128, 500000), (256, 64, 8, 128, 500000), (64, 32, 8, 128, 500000), (17, 4, 2, 64, 10000),
               (9, 8, 2, 256, 10000), (9, 3, 1, 96, 500000),
               (5, 2, 2, 6, 10000), (3, 2, 0, 128, 500000)]
+ROPE_CASES += [(1031, 16, 16, 64, 10000), (1025, 8, 2, 128, 500000)]   # four tokens per step
 
 
 @pytest.mark.parametrize("dt", F8, ids=dt_id)

@@ -386,6 +386,11 @@ for _ in range(3):
 
 # Llama-3-70B and 405B heads; head_dim 256 and the largest accepted, 512
 ROPE_CASES += [(256, 64, 8, 128, 500000), (16, 128, 8, 128, 500000), (9, 8, 2, 256, 10000), (3, 2, 1, 512, 10000)]
+# several tokens per workgroup step (four or two, with one to three left for
+# the last step, no K rows, and the fewest tokens that take it), and rows of
+# 512 threads' chunks, the longest among them
+ROPE_CASES += [(1031, 16, 16, 64, 10000), (1025, 3, 1, 96, 500000), (2050, 8, 0, 64, 500000), (1026, 24, 3, 64, 500000),
+               (1281, 32, 8, 128, 500000), (300, 40, 40, 128, 500000), (9, 64, 64, 128, 500000), (9, 64, 32, 128, 500000)]
 
 
 def rope_inputs(dt, T, nq, nkv, hd, seed=51):
@@ -510,6 +515,13 @@ ROPE_KV_CASES = [
     (9, 3, 1, 96, 4, 1),
     (40, 32, 8, 128, 16, 1),
     (5, 2, 0, 128, 3, 0),
+    # several tokens per step, whose context rows lie anywhere; 512-thread rows
+    (1031, 16, 16, 64, 100, 0),
+    (1025, 8, 2, 64, 33, 1),
+    (1281, 32, 8, 128, 700, 0),
+    (1283, 32, 8, 128, 700, 1),
+    (70, 40, 40, 128, 16, 0),
+    (33, 64, 64, 128, 16, 1),
 ]
 for _ in range(2):
     _nq = _ri(1, 32)
