@@ -243,6 +243,16 @@ static int launch(hipFunction_t fn, Hip_Launch_Config * cfg, hipStream_t stream,
 	return 0;
 }
 
+/* the op's kernel that a launch configuration names (0: the main one) */
+static int pick_kernel(Hip_Function * f, unsigned variant, const char * nick, hipFunction_t * out) {
+	*out = variant == 0 ? f->function_handle : (variant <= HIP_NUM_VARIANTS ? f->variant_handles[variant - 1] : NULL);
+	if (!*out) {
+		fprintf(stderr, "hip backend: op %s: the launch configuration chose kernel variant %u, which the code object lacks\n", nick, variant);
+		return -1;
+	}
+	return 0;
+}
+
 static int hip_submit_op(Dataflow_Handle * dataflow_handle, Op * op, int stream_id) {
 	const char * nick = op->op_skeleton.header.op_nickname;
 	hipStream_t stream;
@@ -268,13 +278,9 @@ static int hip_submit_op(Dataflow_Handle * dataflow_handle, Op * op, int stream_
 		if (cfg.gridDimX == 0 || cfg.gridDimY == 0 || cfg.gridDimZ == 0) {
 			return 0;
 		}
-		hipFunction_t kernel = f->function_handle;
-		if (cfg.variant != 0) {
-			kernel = cfg.variant <= HIP_NUM_VARIANTS ? f->variant_handles[cfg.variant - 1] : NULL;
-			if (!kernel) {
-				fprintf(stderr, "hip backend: op %s: the launch configuration chose kernel variant %u, which the code object lacks\n", nick, cfg.variant);
-				return -1;
-			}
+		hipFunction_t kernel, then_kernel;
+		if (pick_kernel(f, cfg.variant, nick, &kernel) || pick_kernel(f, cfg.then_variant, nick, &then_kernel)) {
+			return -1;
 		}
 		Hip_Context * hc = (Hip_Context *) dataflow_handle->ctx;
 		if (f->function_config.shares_module_scratch && hc->two_pass_stream != HIP_NO_STREAM && hc->two_pass_stream != stream_id) {
@@ -287,7 +293,7 @@ static int hip_submit_op(Dataflow_Handle * dataflow_handle, Op * op, int stream_
 			HIP_CHECK_RET(hipEventRecord(hc->two_pass_event, prev), -1, "ordering op %s after the previous scratch user", nick);
 			HIP_CHECK_RET(hipStreamWaitEvent(stream, hc->two_pass_event, 0), -1, "ordering op %s after the previous scratch user", nick);
 		}
-		if (launch(kernel, &cfg, stream, op)) {
+		if (launch(kernel, &cfg, stream, op) || (cfg.then_variant && launch(then_kernel, &cfg, stream, op))) {
 			fprintf(stderr, "hip backend: op %s: kernel launch failed\n", nick);
 			return -1;
 		}

@@ -386,6 +386,13 @@ static int smx_config(Hip_Launch_Config * c, Dataflow_Handle * h, Hip_Function *
 		c->variant = kernel == SMX_ROWS ? HIP_VARIANT_ROWS : HIP_VARIANT_WIDE_ROWS;
 		return 0;
 	}
+	if (kernel == SMX_SPLIT) {
+		const int slices = smx_split_slices(n_rows, smx_split_sets(n_cols, (int) elem, ptr_bits(x), ptr_bits(out)));
+		set_1d(c, (unsigned) (MY_CEIL(n_rows, SMX_SPLIT_XCDS) * SMX_SPLIT_XCDS * slices), SMX_THREADS, 0);
+		c->variant = HIP_VARIANT_SPLIT;
+		c->then_variant = HIP_VARIANT_SPLIT_OUT;
+		return 0;
+	}
 	/* persistent over rows: one workgroup of SMX_THREADS per CU (a row fills
 	 * its VGPRs and half its LDS) */
 	const long grid = MY_MIN((long) n_rows, (long) dev(h)->cu_count);

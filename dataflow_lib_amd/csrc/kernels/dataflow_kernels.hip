@@ -8,5 +8,6 @@
 #include "swiglu.hip"
 #include "softmax_xent.hip"
 #include "softmax_rows.hip"
+#include "softmax_split.hip"
 #include "gather_scatter.hip"
 #include "fp8_ops.hip"

@@ -47,6 +47,14 @@
 #define SMX_WIDE_ROWS_CH 16
 #define SMX_ROWS_PER_WG 4
 
+/* softmax / cross-entropy, "_split" kernels: few rows of many chunks, each over
+ * up to SMX_SPLIT_MAX workgroups of SMX_THREADS, a slice being up to
+ * SMX_SPLIT_K sets of SMX_THREADS chunks */
+#define SMX_SPLIT_ROWS 64
+#define SMX_SPLIT_MAX 16
+#define SMX_SPLIT_K 4
+#define SMX_SPLIT_XCDS 8
+
 /* RoPE, head_dim <= 512. Vector path: one ROPE_SLOT_THREADS workgroup per
  * token at a time (persistent over tokens, next token prefetched), thread t
  * owning Q chunks t + 256 j (j < ROPE_QJ) and K chunks t + 256 j (j < ROPE_KJ)
@@ -219,7 +227,28 @@ GEOM_FN int smx_rows_waves(int ch, int n_rows, int n_cols, int elem_bytes, unsig
 	return g;
 }
 
+/* "_split" kernels: a row's sets of SMX_THREADS chunks, and the workgroups a
+ * row is split over: as many as give the chip a workgroup per CU */
+GEOM_FN int smx_split_sets(int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
+	return (smx_rows_chunks(n_cols, elem_bytes, x, out) + SMX_THREADS - 1) / SMX_THREADS;
+}
+GEOM_FN int smx_split_slices(int n_rows, int sets) {
+	int s = 256 / n_rows;
+	if (s > SMX_SPLIT_MAX) s = SMX_SPLIT_MAX;
+	if (s > sets) s = sets;
+	if (s < 1) return 1;
+	/* no more than the slices' sets need */
+	const int k = (sets + s - 1) / s;
+	return (sets + k - 1) / k;
+}
+
 /* Which kernel a softmax / cross-entropy call takes. In order:
+ * - SMX_SPLIT for at most SMX_SPLIT_ROWS rows of more than seven sets of
+ *   SMX_THREADS chunks, in slices of at most SMX_SPLIT_K: two launches, so
+ *   shorter rows stay on one CU (softmax 16 x 65536 bf16 9.5 -> 7.9 us, but
+ *   16 x 50257 8.9 -> 10.6), and so do more rows, whose slices are long and
+ *   whose maxima are then found too often over (128 x 128256 20.8 us either
+ *   way, fp16 21.9 -> 27.0);
  * - SMX_LONG_ROWS for aligned 16-bit rows of 17 to 20 chunks per thread;
  * - SMX_ROWS (8 chunks per thread) while the row needs at most 8 waves (16-bit)
  *   or 4 (fp32), so that at least two rows share a CU, and up to 16 waves when
@@ -241,12 +270,18 @@ GEOM_FN int smx_rows_waves(int ch, int n_rows, int n_cols, int elem_bytes, unsig
 #define SMX_ROWS 1
 #define SMX_WIDE_ROWS 2
 #define SMX_LONG_ROWS 3
+#define SMX_SPLIT 4
 #define SMX_FEW_ROWS 256   /* no more rows than CUs: each row has a CU to itself */
 GEOM_FN int smx_kernel_for(int n_rows, int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
 	const int chunks = smx_rows_chunks(n_cols, elem_bytes, x, out);
 	const int few = n_rows <= SMX_FEW_ROWS;
 	/* the main kernel holds the row in registers too */
 	const int main_regs = ((x | out) & 15ull) == 0ull && ((long) n_cols * elem_bytes) % 16 == 0;
+	if (chunks > 7 * SMX_THREADS && n_rows <= SMX_SPLIT_ROWS) {
+		const int sets = (chunks + SMX_THREADS - 1) / SMX_THREADS;
+		const int slices = smx_split_slices(n_rows, sets);
+		if ((sets + slices - 1) / slices <= SMX_SPLIT_K) return SMX_SPLIT;
+	}
 	if (main_regs && elem_bytes == 2 && chunks > 1024 * SMX_MAXCH && ((long) n_cols * elem_bytes) / 16 <= 1024 * SMX_LONG_MAXCH) return SMX_LONG_ROWS;
 	if (chunks == 0 || chunks > 1024 * SMX_WIDE_ROWS_CH) return SMX_MAIN;
 	if (elem_bytes == 1) {

@@ -27,19 +27,24 @@ struct SmxChunk {
 	static constexpr int N = VecOf<T>::N;
 	typedef R16 raw;
 	__device__ static __forceinline__ raw load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) { return buf_load16_nt(r, voff, soff); }
+	/* for data that other workgroups of the launch read too */
+	__device__ static __forceinline__ raw load_again(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) { return buf_load16(r, voff, soff); }
 	__device__ static __forceinline__ void unpack(const raw & r, float * f) { unpack16<T>(r, f); }
 };
 template <typename T>
 struct SmxChunkFp8 {
 	static constexpr int N = 8;
 	typedef R8 raw;
-	__device__ static __forceinline__ raw load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-		const u32x2_v v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, BUF_AUX_NT);
+	template <int AUX>
+	__device__ static __forceinline__ raw load_aux(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+		const u32x2_v v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, AUX);
 		raw o;
 		o.w[0] = v.x;
 		o.w[1] = v.y;
 		return o;
 	}
+	__device__ static __forceinline__ raw load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) { return load_aux<BUF_AUX_NT>(r, voff, soff); }
+	__device__ static __forceinline__ raw load_again(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) { return load_aux<0>(r, voff, soff); }
 	__device__ static __forceinline__ void unpack(const raw & r, float * f) { unpack8_fp8<T>(r, f); }
 	__device__ static __forceinline__ void opaque(raw & r) { reg_barrier8(r); }
 };
@@ -124,7 +129,7 @@ __device__ unsigned int g_smx_group_done[(SMX_GROUPS + 1) * SMX_GROUP_STRIDE];
 __device__ double g_smx_group_sum[SMX_GROUPS];
 
 struct SmxGroup {
-	int first, count, index, n_groups;
+	int first, count, index, n_groups;   /* workgroups */
 	__device__ __forceinline__ SmxGroup() {
 		const int wg = (int) blockIdx.x, n = (int) gridDim.x;
 		int per = (n + SMX_GROUPS - 1) / SMX_GROUPS;

@@ -54,8 +54,10 @@ typedef struct hip_device_info {
 #define HIP_VARIANT_WIDE_ROWS 2   /* "_wide_rows" */
 #define HIP_VARIANT_LONG_ROWS 3   /* "_long_rows" */
 #define HIP_VARIANT_MULTI 4       /* "_multi" */
-#define HIP_NUM_VARIANTS 4
-#define HIP_VARIANT_SUFFIXES {"_rows", "_wide_rows", "_long_rows", "_multi"}
+#define HIP_VARIANT_SPLIT 5       /* "_split" */
+#define HIP_VARIANT_SPLIT_OUT 6   /* "_split_out" */
+#define HIP_NUM_VARIANTS 6
+#define HIP_VARIANT_SUFFIXES {"_rows", "_wide_rows", "_long_rows", "_multi", "_split", "_split_out"}
 
 typedef struct hip_function_config {
 	int func_max_smem;
@@ -82,6 +84,9 @@ typedef struct hip_launch_config {
 	/* which of the op's kernels to launch: 0 function_handle, i > 0
 	 * variant_handles[i - 1] */
 	unsigned int variant;
+	/* a second kernel (a variant, 0: none) launched right after it with the
+	 * same geometry and parameters */
+	unsigned int then_variant;
 } Hip_Launch_Config;
 
 typedef struct hip_function Hip_Function;

@@ -10,7 +10,7 @@
 
 int main(void) {
 	static const unsigned long long offsets[] = {0, 16, 64, 112, 2, 6, 34, 128, 4, 12, 8, 1, 5};
-	static const int row_counts[] = {1, 200, 257, 5000};
+	static const int row_counts[] = {1, 7, 64, 200, 257, 5000};
 	const int n_off = (int) (sizeof(offsets) / sizeof(offsets[0]));
 	long bad = 0;
 	for (int e = 1; e <= 4; e *= 2) {
@@ -19,7 +19,7 @@ int main(void) {
 		for (int i = 0; i < n_off * n_off; i++) {
 			const unsigned long long x = 4096 + offsets[i / n_off], o = 8192 + offsets[i % n_off];
 			if (x % e || o % oe) continue;
-			for (int n = 1; n < 140000; n += (n < 700 || (n > 130800 && n < 131200)) ? 1 : 1997) {
+			for (int n = 1; n < 540000; n += (n < 700 || (n > 130900 && n < 131100)) ? 1 : 1997) {
 				const int bound = smx_rows_chunks(n, e, x, o);
 				if (!bound) continue;
 				const unsigned line = smx_rows_line(n, e, x, o);
@@ -31,8 +31,15 @@ int main(void) {
 						if (bad++ < 10) printf("elem %d, %d columns, x+%llu out+%llu, row %d: %ld chunks of %d, out %llu\n", e, n, x - 4096, o - 8192, r, need, bound, out & 15);
 					}
 				}
-				for (int k = 0; k < 4; k++) {
+				for (int k = 0; k < 6; k++) {
 					const int kernel = smx_kernel_for(row_counts[k], n, e, x, o);
+					if (kernel == SMX_SPLIT) {
+						const int sets = smx_split_sets(n, e, x, o), s = smx_split_slices(row_counts[k], sets);
+						const int per = (sets + s - 1) / s;
+						if (row_counts[k] > SMX_SPLIT_ROWS || s < 1 || s > SMX_SPLIT_MAX || per > SMX_SPLIT_K || (long) s * per * SMX_THREADS < bound) {
+							if (bad++ < 10) printf("elem %d, %d rows of %d columns: %d slices of %d sets\n", e, row_counts[k], n, s, per);
+						}
+					}
 					if (kernel != SMX_ROWS && kernel != SMX_WIDE_ROWS) continue;
 					const int ch = kernel == SMX_ROWS ? SMX_ROWS_CH : SMX_WIDE_ROWS_CH;
 					const int g = smx_rows_waves(ch, row_counts[k], n, e, x, o);

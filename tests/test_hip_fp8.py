@@ -329,7 +329,7 @@ SMX_SHAPES = [(4, 128256), (3, 1000), (2, 1001), (2, 140000), (5, 64), (1, 1), (
               (300, 32768), (520, 65552), (260, 128256), (2, 131072), (5, 65536), (1100, 128256)]
 # rows of one wave, of several, and of 16 chunks per thread, whose 8-byte
 # chunks reach into the rows beside them; many short rows
-SMX_SHAPES += [(9, 513), (5, 4097), (300, 16383), (3, 49161), (300, 49145), (2, 65529), (2, 130001), (3, 131064), (600, 33)]
+SMX_SHAPES += [(9, 513), (5, 4097), (300, 16383), (3, 49161), (300, 49145), (2, 65529), (2, 130001), (3, 131064), (600, 33), (64, 60000), (70, 100001)]
 # logits placed off 16-byte alignment: the element-wise loop (for (5, 65536),
 # with the long-row path's workgroup size)
 SMX_UNALIGNED = ((2, 1001), (5, 65536))

@@ -747,6 +747,7 @@ def special_logits(dt, shape, seed):
 # the loss sum counts
 ROW_SHAPES = [(9, 2047, 0), (9, 2049, 1), (5, 4088, 0), (5, 4097, 3), (7, 16385, 0), (5, 32761, 1), (5, 32776, 0), (3, 65529, 5),
               (3, 65544, 8), (2, 131001, 0), (2, 131073, 1), (259, 40001, 0), (2051, 200, 0), (523, 65, 7),
+              (17, 57400, 0), (64, 58001, 3), (65, 58000, 0), (1, 200001, 1), (40, 66000, 0),   # few long rows: split over workgroups
               (2, 163840, 0), (2, 163848, 0)]   # the last 16-bit row held in 20 chunks per thread, and one past it
 
 
