@@ -398,6 +398,7 @@ static int smx_config(Hip_Launch_Config * c, Dataflow_Handle * h, Hip_Function *
 	const long grid = MY_MIN((long) n_rows, (long) dev(h)->cu_count);
 	set_1d(c, (unsigned) grid, SMX_THREADS, 0);
 	if (kernel == SMX_LONG_ROWS) c->variant = HIP_VARIANT_LONG_ROWS;
+	else if (kernel == SMX_ANY_ROWS) c->variant = HIP_VARIANT_ANY_ROWS;
 	return 0;
 }
 

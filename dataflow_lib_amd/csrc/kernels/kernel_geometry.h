@@ -243,10 +243,11 @@ GEOM_FN int smx_split_slices(int n_rows, int sets) {
 }
 
 /* Which kernel a softmax / cross-entropy call takes. In order:
- * - SMX_SPLIT for at most SMX_SPLIT_ROWS rows of more than seven sets of
- *   SMX_THREADS chunks, in slices of at most SMX_SPLIT_K: two launches, so
- *   shorter rows stay on one CU (softmax 16 x 65536 bf16 9.5 -> 7.9 us, but
- *   16 x 50257 8.9 -> 10.6), and so do more rows, whose slices are long and
+ * - SMX_SPLIT for at most SMX_SPLIT_ROWS rows (half as many of 8 sets) of more
+ *   than seven (fp32: eight) sets of SMX_THREADS chunks, in slices of at most
+ *   SMX_SPLIT_K: two launches, so shorter rows stay on one CU (softmax 16 x
+ *   65536 bf16 9.5 -> 7.9 us, but 16 x 50257 8.9 -> 10.6, fp32 64 x 32000 7.6
+ *   -> 8.5), and so do more rows, whose slices are long and
  *   whose maxima are then found too often over (128 x 128256 20.8 us either
  *   way, fp16 21.9 -> 27.0);
  * - SMX_LONG_ROWS for aligned 16-bit rows of 17 to 20 chunks per thread;
@@ -261,6 +262,8 @@ GEOM_FN int smx_split_slices(int n_rows, int sets) {
  *   next on the same CU (1024 x 100000 bf16 78.5 us, wide 98.3; 4096 x 32000
  *   fp32 169.4, wide 184.1), unless they are unaligned, which it does not
  *   hold in registers (1024 x 128257 bf16 557 us, wide 116);
+ * - unaligned rows of more than 16 chunks per thread to SMX_ANY_ROWS, which
+ *   streams them as the main kernel does aligned ones;
  * - fp8 logits the same way: 12 waves of 8 chunks still share a CU with
  *   another row (1024 x 48000 27.7 us, wide 30.3; 1024 x 50256 43.0, wide
  *   31.6), and the main kernel overlaps rows from some 512 on (300 x 128256
@@ -271,19 +274,21 @@ GEOM_FN int smx_split_slices(int n_rows, int sets) {
 #define SMX_WIDE_ROWS 2
 #define SMX_LONG_ROWS 3
 #define SMX_SPLIT 4
+#define SMX_ANY_ROWS 5
 #define SMX_FEW_ROWS 256   /* no more rows than CUs: each row has a CU to itself */
 GEOM_FN int smx_kernel_for(int n_rows, int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
 	const int chunks = smx_rows_chunks(n_cols, elem_bytes, x, out);
 	const int few = n_rows <= SMX_FEW_ROWS;
 	/* the main kernel holds the row in registers too */
 	const int main_regs = ((x | out) & 15ull) == 0ull && ((long) n_cols * elem_bytes) % 16 == 0;
-	if (chunks > 7 * SMX_THREADS && n_rows <= SMX_SPLIT_ROWS) {
+	if (chunks > (elem_bytes == 4 ? 8 : 7) * SMX_THREADS && n_rows <= (chunks > 8 * SMX_THREADS ? SMX_SPLIT_ROWS : SMX_SPLIT_ROWS / 2)) {
 		const int sets = (chunks + SMX_THREADS - 1) / SMX_THREADS;
 		const int slices = smx_split_slices(n_rows, sets);
 		if ((sets + slices - 1) / slices <= SMX_SPLIT_K) return SMX_SPLIT;
 	}
 	if (main_regs && elem_bytes == 2 && chunks > 1024 * SMX_MAXCH && ((long) n_cols * elem_bytes) / 16 <= 1024 * SMX_LONG_MAXCH) return SMX_LONG_ROWS;
-	if (chunks == 0 || chunks > 1024 * SMX_WIDE_ROWS_CH) return SMX_MAIN;
+	if (chunks == 0) return SMX_MAIN;
+	if (chunks > 1024 * SMX_WIDE_ROWS_CH) return (main_regs || elem_bytes == 1) ? SMX_MAIN : SMX_ANY_ROWS;
 	if (elem_bytes == 1) {
 		if (chunks <= (few ? 1024 : 768) * SMX_ROWS_CH) return SMX_ROWS;
 		return (chunks <= 1024 * SMX_ROWS_CH || n_rows <= 2 * SMX_FEW_ROWS || !f8_smx_pf_ok(n_cols)) ? SMX_WIDE_ROWS : SMX_MAIN;

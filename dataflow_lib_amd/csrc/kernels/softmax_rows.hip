@@ -51,35 +51,6 @@ struct SmxChunkFp8 {
 template <> struct SmxChunk<fp8e4m3_t> : SmxChunkFp8<fp8e4m3_t> {};
 template <> struct SmxChunk<fp8e5m2_t> : SmxChunkFp8<fp8e5m2_t> {};
 
-/* The chunks that cover a row: the window starts at the 128-byte line (16-byte
- * chunk, where input and output lie differently within their lines) that
- * holds the row's first element, so that every wave's loads and stores are
- * whole lines however long the rows are. Elements [h, end) of the window are
- * the row's; the others belong to the neighbouring rows, are read with it (a
- * chunk never crosses a page) and never written. */
-struct SmxWindow {
-	const char * in;
-	char * out;
-	uint32_t h, end;
-	int chunks;
-};
-
-template <typename T, typename TO>
-__device__ __forceinline__ SmxWindow smx_window(const T * X, TO * out, int n_cols, int row) {
-	const int64_t first = (int64_t) row * n_cols;   /* the row's first element */
-	const uint64_t a = (uint64_t) (uintptr_t) (X + first);
-	/* outputs of another size: X and out are 16-byte aligned (smx_rows_chunks),
-	 * so the window's first element is a chunk's first in out too */
-	const uint64_t mask = smx_rows_line(n_cols, (int) sizeof(T), (unsigned long long) (uintptr_t) X, (unsigned long long) (uintptr_t) out);
-	SmxWindow w;
-	w.h = (uint32_t) (a & mask) / (uint32_t) sizeof(T);
-	w.in = reinterpret_cast<const char *>(a & ~mask);
-	w.out = reinterpret_cast<char *>(out + (first - (int64_t) w.h));
-	w.end = w.h + (uint32_t) n_cols;
-	w.chunks = (int) ((w.end + SmxChunk<T>::N - 1) / SmxChunk<T>::N);
-	return w;
-}
-
 /* reductions over the `g` waves of a row, the waves' partials combined from
  * one LDS read per lane (16 cells, then the row of 16 lanes) in a fixed order */
 __device__ __forceinline__ float row16_max(float v) {

@@ -671,6 +671,36 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 	WAIT_VMEM_ALL();
 }
 
+/* The chunks that cover a row: the window starts at the 128-byte line (16-byte
+ * chunk, where input and output lie differently within their lines) that
+ * holds the row's first element, so that every wave's loads and stores are
+ * whole lines however long the rows are. Elements [h, end) of the window are
+ * the row's; the others belong to the neighbouring rows, are read with it (a
+ * chunk never crosses a page) and never written. */
+struct SmxWindow {
+	const char * in;
+	char * out;
+	uint32_t h, end;
+	int chunks;
+};
+
+template <typename T, typename TO>
+__device__ __forceinline__ SmxWindow smx_window(const T * X, TO * out, int n_cols, int row) {
+	const int64_t first = (int64_t) row * n_cols;   /* the row's first element */
+	const uint64_t a = (uint64_t) (uintptr_t) (X + first);
+	/* outputs of another size: X and out are 16-byte aligned (smx_rows_chunks),
+	 * so the window's first element is a chunk's first in out too */
+	const uint64_t mask = smx_rows_line(n_cols, (int) sizeof(T), (unsigned long long) (uintptr_t) X, (unsigned long long) (uintptr_t) out);
+	SmxWindow w;
+	w.h = (uint32_t) (a & mask) / (uint32_t) sizeof(T);
+	w.in = reinterpret_cast<const char *>(a & ~mask);
+	w.out = reinterpret_cast<char *>(out + (first - (int64_t) w.h));
+	w.end = w.h + (uint32_t) n_cols;
+	constexpr int N = sizeof(T) == 1 ? 8 : VecOf<T>::N;   /* SmxChunk */
+	w.chunks = (int) ((w.end + N - 1) / N);
+	return w;
+}
+
 /* any row length / alignment: three passes over global memory per row */
 template <typename T, typename TO, bool FUSED>
 __device__ __forceinline__ void smx_stream(int n_rows, int n_cols, const T * X, TO * out, const uint32_t * labels, float * loss) {
@@ -711,7 +741,8 @@ __device__ __forceinline__ void smx_stream(int n_rows, int n_cols, const T * X, 
 }
 
 /* Rows longer than the register paths hold (more than SMX_MAXCH 16-byte
- * chunks per thread, SMX_LONG_MAXCH for 16-bit rows), 16-byte aligned: streaming passes over the row with
+ * chunks per thread, SMX_LONG_MAXCH for 16-bit rows), 16-byte aligned, or
+ * (RAGGED, kernels of their own) at any alignment that input and output share: streaming passes over the row with
  * 16-byte accesses. The first pass finds the row max and, online, the sum of
  * exp(x - m) over the unrounded differences (each thread keeps its running
  * max and its sum against it, rescaled when the max grows; mref = 0 while the
@@ -724,7 +755,7 @@ __device__ __forceinline__ void smx_stream(int n_rows, int n_cols, const T * X, 
  * the later passes find the row in cache where they can. The labelled logit
  * is taken from the first pass's registers by the thread holding it (the last
  * pass may overwrite the row in place). */
-template <typename T, bool FUSED>
+template <typename T, bool FUSED, bool RAGGED = false>
 __device__ __forceinline__ void smx_stream_vec(int n_rows, int n_cols, const T * X, T * out, const uint32_t * labels, float * loss) {
 	constexpr int U = 4;
 	constexpr int VEC = VecOf<T>::N;
@@ -738,7 +769,11 @@ __device__ __forceinline__ void smx_stream_vec(int n_rows, int n_cols, const T *
 	 * first pass's working set stays small (measured at 4096 x 151936, which
 	 * the 20-chunk register path holds now: bf16 fused 660.9 -> 591.1 us,
 	 * softmax 651.1 -> 563.5 us). The outputs are bit-identical; the loss sum is rescaled
-	 * at other chunks, so a loss can differ in its last bits. */
+	 * at other chunks, so a loss can differ in its last bits. RAGGED rows hold
+	 * as much, though some of their kernels then spill a few registers: with
+	 * a group less fused fp32 1024 x 128257 took 235 us instead of 220. They
+	 * have kernels of their own because the windows' bounds made the aligned
+	 * ones spill (fused fp32 512 x 200000 167 -> 188 us). */
 	constexpr int HG = sizeof(T) == 4 ? 4 : (FUSED ? 3 : 4);
 	constexpr int UH = sizeof(T) == 4 ? U : 2;   /* chunks per held group */
 	__shared__ float slots[32];
@@ -746,8 +781,6 @@ __device__ __forceinline__ void smx_stream_vec(int n_rows, int n_cols, const T *
 	__shared__ int nextcell;
 	const int tid = threadIdx.x;
 	const int nt = blockDim.x;
-	const int nv = n_cols / VEC;
-	const uint32_t row_bytes = (uint32_t) n_cols * (uint32_t) sizeof(T);
 	/* Rows are handed out as workgroups free up: each workgroup's first row
 	 * is its block index, every later one a ticket t of the launch's row
 	 * counter, row grid + t. Thread 0 requests the ticket for the next row
@@ -761,12 +794,24 @@ __device__ __forceinline__ void smx_stream_vec(int n_rows, int n_cols, const T *
 	 * 4096 x 151936 softmax 566.3 -> 557.1 us, outputs identical. */
 	int row = blockIdx.x;
 	while (row < n_rows) {
-		const __amdgpu_buffer_rsrc_t rin = make_rsrc(X + (long) row * n_cols, row_bytes);
-		const __amdgpu_buffer_rsrc_t rout = make_rsrc(out + (long) row * n_cols, row_bytes);
+		SmxWindow w;
+		if constexpr (RAGGED) w = smx_window<T, T>(X, out, n_cols, row);
+		else {
+			w.in = reinterpret_cast<const char *>(X + (long) row * n_cols);
+			w.out = reinterpret_cast<char *>(out + (long) row * n_cols);
+			w.h = 0u;
+			w.chunks = n_cols / VEC;
+		}
+		const int nv = w.chunks;
+		const __amdgpu_buffer_rsrc_t rin = make_rsrc(w.in, (uint32_t) nv * 16u);
+		const __amdgpu_buffer_rsrc_t rout = make_rsrc(w.out, (uint32_t) nv * 16u);
 		const uint32_t lab = FUSED ? labels[row] : 0xffffffffu;
 		const bool lab_ok = FUSED && lab < (uint32_t) n_cols;
-		const int c_lab = lab_ok ? (int) (lab / VEC) : -1;
-		const int le = (int) (lab % VEC);
+		const int c_lab = lab_ok ? (int) ((lab + w.h) / VEC) : -1;
+		const int le = (int) ((lab + w.h) % VEC);
+		/* whether chunk c holds elements outside the row, and which */
+		auto partial = [&](int c) { return (uint32_t) c * VEC < w.h || (uint32_t) (c + 1) * VEC > w.end; };
+		auto outside = [&](int c, int e) { return (uint32_t) (c * VEC + e) < w.h || (uint32_t) (c * VEC + e) >= w.end; };
 		/* pass 1: max and the online sum of exp(x - m) */
 		float m = -__builtin_inff(), mref = 0.0f, s = 0.0f;
 		auto pass1 = [&](auto & v, int base) {
@@ -777,9 +822,16 @@ __device__ __forceinline__ void smx_stream_vec(int n_rows, int n_cols, const T *
 			for (int k = 0; k < U; k++) {
 				const int c = base + k * nt + tid;
 				unpack16<T>(v[k], f[k]);
+				if constexpr (RAGGED) {
+					if (partial(c)) {
+#pragma unroll
+						for (int e = 0; e < VEC; e++)
+							if (outside(c, e)) f[k][e] = -__builtin_inff();
+					}
+				}
 #pragma unroll
 				for (int e = 0; e < VEC; e++) {
-					if (c >= nv) f[k][e] = -__builtin_inff();
+					if (!RAGGED && c >= nv) f[k][e] = -__builtin_inff();
 					cm = fmaxf(cm, f[k][e]);
 				}
 			}
@@ -845,9 +897,15 @@ __device__ __forceinline__ void smx_stream_vec(int n_rows, int n_cols, const T *
 				constexpr int U = sizeof(v) / sizeof(R16);
 #pragma unroll
 				for (int k = 0; k < U; k++) {
-					if (base + k * nt + tid < nv) {
+					const int c = base + k * nt + tid;
+					if (c < nv) {
 						float f[VEC];
 						unpack16<T>(v[k], f);
+						if (RAGGED && partial(c)) {
+#pragma unroll
+							for (int e = 0; e < VEC; e++)
+								if (outside(c, e)) f[e] = -__builtin_inff();
+						}
 #pragma unroll
 						for (int e = 0; e < VEC; e++) sd += exp_fast(rnd_in<T>(f[e] - mx));
 					}
@@ -884,7 +942,14 @@ __device__ __forceinline__ void smx_stream_vec(int n_rows, int n_cols, const T *
 					f[le] -= 1.0f;
 					o = pack16<T>(f);
 				}
-				buf_store16_nt(rout, (uint32_t) c * 16u, 0, o);
+				if (!RAGGED || !partial(c)) buf_store16_nt(rout, (uint32_t) c * 16u, 0, o);
+				else if (c < nv) {
+					T * p = reinterpret_cast<T *>(w.out);
+					unpack16<T>(o, f);
+#pragma unroll
+					for (int e = 0; e < VEC; e++)
+						if (!outside(c, e)) p[c * VEC + e] = from_f<T>(f[e]);
+				}
 			}
 		};
 #pragma unroll
@@ -933,6 +998,24 @@ __device__ __forceinline__ void smx(int n_rows, int n_cols, const T * X, TO * ou
 		T * p = pred_logits + r * (long) n_cols + lab;                                                                 \
 		*p = from_f<T>(to_f(*p) - 1.0f);                                                                               \
 	}
+
+/* Rows past the "_rows" kernels that are not 16-byte aligned. 512 x 200001:
+ * bf16 softmax 438 -> 109 us, fused 480 -> 115 (410 MB: 3.8 / 3.6 TB/s), fp32
+ * 585 -> 169 and 512 -> 190, against the element path. */
+#define SMX_ANY_KERNELS(SUFFIX, PSUFFIX, T)                                                                            \
+	extern "C" __global__ void __launch_bounds__(SMX_THREADS) softmax_##PSUFFIX##_kernel_any_rows(int n_rows,          \
+			int n_cols, T * X, T * out) {                                                                              \
+		smx_stream_vec<T, false, true>(n_rows, n_cols, X, out, nullptr, nullptr);                                      \
+		smx_launch_end<false>(n_rows, nullptr, nullptr);                                                               \
+	}                                                                                                                  \
+	extern "C" __global__ void __launch_bounds__(SMX_THREADS) softmax_cross_entropy_loss_##SUFFIX##_kernel_any_rows(   \
+			int n_rows, int n_cols, T * logits, uint32_t * labels, float * loss, float * mean_loss) {                  \
+		smx_stream_vec<T, true, true>(n_rows, n_cols, logits, logits, labels, loss);                                   \
+		smx_launch_end<true>(n_rows, loss, mean_loss);                                                                 \
+	}
+SMX_ANY_KERNELS(fp32, fp32_fp32, float)
+SMX_ANY_KERNELS(fp16, fp16_fp16, f16_t)
+SMX_ANY_KERNELS(bf16, bf16_bf16, bf16_t)
 
 /* 16-bit rows of 131,080 to 163,840 columns, held whole: 4096 x 151936 bf16
  * fused 594 -> 461 us, softmax 557 -> 441 us (2.49 GB: 5.4 / 5.65 TB/s) against

@@ -56,8 +56,9 @@ typedef struct hip_device_info {
 #define HIP_VARIANT_MULTI 4       /* "_multi" */
 #define HIP_VARIANT_SPLIT 5       /* "_split" */
 #define HIP_VARIANT_SPLIT_OUT 6   /* "_split_out" */
-#define HIP_NUM_VARIANTS 6
-#define HIP_VARIANT_SUFFIXES {"_rows", "_wide_rows", "_long_rows", "_multi", "_split", "_split_out"}
+#define HIP_VARIANT_ANY_ROWS 7    /* "_any_rows" */
+#define HIP_NUM_VARIANTS 7
+#define HIP_VARIANT_SUFFIXES {"_rows", "_wide_rows", "_long_rows", "_multi", "_split", "_split_out", "_any_rows"}
 
 typedef struct hip_function_config {
 	int func_max_smem;

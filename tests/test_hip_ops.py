@@ -748,6 +748,7 @@ def special_logits(dt, shape, seed):
 ROW_SHAPES = [(9, 2047, 0), (9, 2049, 1), (5, 4088, 0), (5, 4097, 3), (7, 16385, 0), (5, 32761, 1), (5, 32776, 0), (3, 65529, 5),
               (3, 65544, 8), (2, 131001, 0), (2, 131073, 1), (259, 40001, 0), (2051, 200, 0), (523, 65, 7),
               (17, 57400, 0), (64, 58001, 3), (65, 58000, 0), (1, 200001, 1), (40, 66000, 0),   # few long rows: split over workgroups
+              (67, 131201, 0), (65, 163901, 3), (300, 70001, 1),   # unaligned rows past 16 chunks per thread (fp32: the last)
               (2, 163840, 0), (2, 163848, 0)]   # the last 16-bit row held in 20 chunks per thread, and one past it
 
 
@@ -878,10 +879,12 @@ def shifted_logits(dt, shape, seed):
 
 
 SHIFTED_SHAPES = [(6, 128256), (6, 151936), (6, 1001)]   # register path (16-bit), streaming vector path, element path
+# the same lengths where there are too many rows to split them over workgroups
+WHOLE_ROW_SHAPES = [(66, 128256), (66, 151936)]
 
 
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
-@pytest.mark.parametrize("shape", SHIFTED_SHAPES, ids=lambda s: "%dx%d" % s)
+@pytest.mark.parametrize("shape", SHIFTED_SHAPES + WHOLE_ROW_SHAPES, ids=lambda s: "%dx%d" % s)
 def test_fused_loss_on_shifted_rows(hdl, dt, shape):
     from dataflow_lib_amd import api
     n_rows, n_cols = shape
