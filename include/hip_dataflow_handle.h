@@ -123,8 +123,8 @@ typedef int (*Hip_Set_Func_Attribute)(Dataflow_Handle * dataflow_handle, Hip_Fun
  * CUDA backend keeps its CUcontext there). The device id comes first, so ctx
  * still reads as the device id. Functions flagged shares_module_scratch keep
  * per-launch state in their code object's module-scope memory (the RMSNorm
- * dW ops their partial rows; the 16-bit and fp32 softmax and fused
- * cross-entropy their row counter and finished-workgroup count), so the
+ * dW ops their partial rows; the softmax and fused cross-entropy their row
+ * counter, finished-workgroup counts and the sums of split rows), so the
  * handle orders them across its streams: such an op submitted on another
  * stream than the previous one first waits for everything then queued on
  * that stream (an event recorded only when the stream changes, so
