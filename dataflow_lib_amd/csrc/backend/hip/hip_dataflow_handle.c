@@ -253,6 +253,43 @@ static int pick_kernel(Hip_Function * f, unsigned variant, const char * nick, hi
 	return 0;
 }
 
+/* an op's launches, ordered after the previous user of the module scratch (the
+ * caller holds two_pass_lock for an op that uses it) */
+static int launch_kernels(Dataflow_Handle * dataflow_handle, Hip_Context * hc, Hip_Function * f, Hip_Launch_Config * cfg,
+						  hipFunction_t kernel, hipFunction_t then_kernel, hipStream_t stream, int stream_id, Op * op) {
+	const char * nick = op->op_skeleton.header.op_nickname;
+	if (f->function_config.shares_module_scratch && hc->two_pass_stream != HIP_NO_STREAM && hc->two_pass_stream != stream_id) {
+		/* the previous op using the module scratch ran on another stream:
+		 * wait for that stream's queued work */
+		hipStream_t prev;
+		if (resolve_stream(dataflow_handle, hc->two_pass_stream, &prev, nick)) {
+			return -1;
+		}
+		HIP_CHECK_RET(hipEventRecord(hc->two_pass_event, prev), -1, "ordering op %s after the previous scratch user", nick);
+		HIP_CHECK_RET(hipStreamWaitEvent(stream, hc->two_pass_event, 0), -1, "ordering op %s after the previous scratch user", nick);
+	}
+	if (launch(kernel, cfg, stream, op) || (cfg->then_variant && launch(then_kernel, cfg, stream, op))) {
+		fprintf(stderr, "hip backend: op %s: kernel launch failed\n", nick);
+		return -1;
+	}
+	if (f->function_config.shares_module_scratch) {
+		hc->two_pass_stream = stream_id;
+	}
+	if (f->finish_function_handle) {
+		Hip_Launch_Config fcfg;
+		memset(&fcfg, 0, sizeof(fcfg));
+		if (f->set_finish_launch_config(&fcfg, dataflow_handle, f, op)) {
+			fprintf(stderr, "hip backend: op %s: the second kernel's launch configuration rejected these arguments\n", nick);
+			return -1;
+		}
+		if (fcfg.gridDimX && fcfg.gridDimY && fcfg.gridDimZ && launch(f->finish_function_handle, &fcfg, stream, op)) {
+			fprintf(stderr, "hip backend: op %s: second kernel launch failed\n", nick);
+			return -1;
+		}
+	}
+	return 0;
+}
+
 static int hip_submit_op(Dataflow_Handle * dataflow_handle, Op * op, int stream_id) {
 	const char * nick = op->op_skeleton.header.op_nickname;
 	hipStream_t stream;
@@ -283,36 +320,11 @@ static int hip_submit_op(Dataflow_Handle * dataflow_handle, Op * op, int stream_
 			return -1;
 		}
 		Hip_Context * hc = (Hip_Context *) dataflow_handle->ctx;
-		if (f->function_config.shares_module_scratch && hc->two_pass_stream != HIP_NO_STREAM && hc->two_pass_stream != stream_id) {
-			/* the previous op using the module scratch ran on another stream:
-			 * wait for that stream's queued work */
-			hipStream_t prev;
-			if (resolve_stream(dataflow_handle, hc->two_pass_stream, &prev, nick)) {
-				return -1;
-			}
-			HIP_CHECK_RET(hipEventRecord(hc->two_pass_event, prev), -1, "ordering op %s after the previous scratch user", nick);
-			HIP_CHECK_RET(hipStreamWaitEvent(stream, hc->two_pass_event, 0), -1, "ordering op %s after the previous scratch user", nick);
-		}
-		if (launch(kernel, &cfg, stream, op) || (cfg.then_variant && launch(then_kernel, &cfg, stream, op))) {
-			fprintf(stderr, "hip backend: op %s: kernel launch failed\n", nick);
-			return -1;
-		}
-		if (f->function_config.shares_module_scratch) {
-			hc->two_pass_stream = stream_id;
-		}
-		if (f->finish_function_handle) {
-			Hip_Launch_Config fcfg;
-			memset(&fcfg, 0, sizeof(fcfg));
-			if (f->set_finish_launch_config(&fcfg, dataflow_handle, f, op)) {
-				fprintf(stderr, "hip backend: op %s: the second kernel's launch configuration rejected these arguments\n", nick);
-				return -1;
-			}
-			if (fcfg.gridDimX && fcfg.gridDimY && fcfg.gridDimZ && launch(f->finish_function_handle, &fcfg, stream, op)) {
-				fprintf(stderr, "hip backend: op %s: second kernel launch failed\n", nick);
-				return -1;
-			}
-		}
-		return 0;
+		const bool shared = f->function_config.shares_module_scratch;
+		if (shared) pthread_mutex_lock(&hc->two_pass_lock);
+		const int ret = launch_kernels(dataflow_handle, hc, f, &cfg, kernel, then_kernel, stream, stream_id, op);
+		if (shared) pthread_mutex_unlock(&hc->two_pass_lock);
+		return ret;
 	}
 
 	if (!f->hip_external_func) {
@@ -546,6 +558,7 @@ int init_hip_dataflow_handle(Dataflow_Handle * dataflow_handle, ComputeType comp
 	Hip_Context * hc = (Hip_Context *) dataflow_handle->ctx;
 	hc->device_id = device_id;
 	hc->two_pass_stream = HIP_NO_STREAM;
+	pthread_mutex_init(&hc->two_pass_lock, NULL);
 	HIP_CHECK_RET(hipEventCreateWithFlags(&hc->two_pass_event, hipEventDisableTiming), init_fail(dataflow_handle), "creating the cross-stream ordering event on device %d", device_id);
 	if (hip_set_device_info((Hip_Device_Info *) dataflow_handle->device_info, device_id)) {
 		fprintf(stderr, "hip backend: reading the properties of device %d failed\n", device_id);
@@ -642,6 +655,7 @@ int destroy_hip_dataflow_handle(Dataflow_Handle * dataflow_handle) {
 	free(dataflow_handle->device_info);
 	Hip_Context * hc = (Hip_Context *) dataflow_handle->ctx;
 	if (hc && hc->two_pass_event) hipEventDestroy(hc->two_pass_event);
+	if (hc) pthread_mutex_destroy(&hc->two_pass_lock);
 	free(dataflow_handle->ctx);
 	dataflow_handle->streams = NULL;
 	dataflow_handle->stream_states = NULL;

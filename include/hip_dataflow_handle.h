@@ -134,6 +134,9 @@ typedef struct hip_context {
 	int device_id;
 	int two_pass_stream;       /* stream id of the last scratch-sharing op, HIP_NO_STREAM before the first */
 	hipEvent_t two_pass_event;
+	/* held while such an op's kernels are launched, so that ops submitted by
+	 * several threads do not come between another op's two launches */
+	pthread_mutex_t two_pass_lock;
 } Hip_Context;
 
 /* ctx_flags is accepted for interface parity and ignored (HIP has no

@@ -792,6 +792,40 @@ def test_softmax_rows_of_any_alignment(hdl, dt, shape):
         check_f32(d.get(pmean, (1,), np.float32), mean, rel=1e-4, what="fused mean loss")
 
 
+def test_split_softmax_from_two_threads(hdl):
+    """A few long rows take two launches that share the code object's memory:
+    submits of two threads on one stream must not come between them. Every
+    output equals the one that a single thread's submit gave."""
+    import threading
+    from dataflow_lib_amd import api
+    n_rows, n_cols, reps = 4, 66000, 60
+    X = [to_storage(normal(171 + k, (n_rows, n_cols), std=2.0 + k), BF16) for k in range(2)]
+    with Dev(hdl) as d:
+        px = [d.put(x) for x in X]
+        po = [[d.empty(x.nbytes) for _ in range(reps + 1)] for x in X]
+        for k in range(2):
+            assert api.submit_softmax(hdl, 0, BF16, BF16, n_rows, n_cols, px[k], po[k][reps]) == 0
+        hdl.sync()
+        bad, start = [], threading.Barrier(2)
+
+        def work(k):
+            start.wait()
+            for i in range(reps):
+                if api.submit_softmax(hdl, 0, BF16, BF16, n_rows, n_cols, px[k], po[k][i]) != 0:
+                    bad.append((k, i))
+
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not bad
+        for k in range(2):
+            want = d.get(po[k][reps], X[k].shape, np.uint16)
+            for i in range(reps):
+                assert np.array_equal(d.get(po[k][i], X[k].shape, np.uint16), want), (k, i)
+
+
 # more rows than workgroups (each walks 2-3 rows with the next row, its label
 # and labelled logit in flight); 32000 and 24576 + 8 columns leave a partial
 # last chunk, 128256 is the Llama-3 vocabulary
