@@ -250,7 +250,11 @@ GEOM_FN int smx_split_slices(int n_rows, int sets) {
  *   -> 8.5), and so do more rows, whose slices are long and
  *   whose maxima are then found too often over (128 x 128256 20.8 us either
  *   way, fp16 21.9 -> 27.0);
- * - SMX_LONG_ROWS for aligned 16-bit rows of 17 to 20 chunks per thread;
+ * - SMX_LONG_ROWS for aligned 16-bit rows of 17 to 20 chunks per thread, by the
+ *   row's own chunks, which that kernel counts and relies on
+ *   (smx_regs_atleast), not by its window's: a window may have up to seven
+ *   more, and with 16 chunks per thread of its own (131,024 to 131,072
+ *   columns) the row is the main kernel's;
  * - SMX_ROWS (8 chunks per thread) while the row needs at most 8 waves (16-bit)
  *   or 4 (fp32), so that at least two rows share a CU, and up to 16 waves when
  *   no two rows have to share one (16 x 50257 bf16: 9.4 us, wide 11.7);
@@ -286,7 +290,8 @@ GEOM_FN int smx_kernel_for(int n_rows, int n_cols, int elem_bytes, unsigned long
 		const int slices = smx_split_slices(n_rows, sets);
 		if ((sets + slices - 1) / slices <= SMX_SPLIT_K) return SMX_SPLIT;
 	}
-	if (main_regs && elem_bytes == 2 && chunks > 1024 * SMX_MAXCH && ((long) n_cols * elem_bytes) / 16 <= 1024 * SMX_LONG_MAXCH) return SMX_LONG_ROWS;
+	const long own = (long) n_cols * elem_bytes / 16;
+	if (main_regs && elem_bytes == 2 && own > 1024 * SMX_MAXCH && own <= 1024 * SMX_LONG_MAXCH) return SMX_LONG_ROWS;
 	if (chunks == 0) return SMX_MAIN;
 	if (chunks > 1024 * SMX_WIDE_ROWS_CH) return (main_regs || elem_bytes == 1) ? SMX_MAIN : SMX_ANY_ROWS;
 	if (elem_bytes == 1) {

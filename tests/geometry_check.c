@@ -1,12 +1,27 @@
-/* The launch rule of the softmax "_rows" kernels against what their rows
- * really take, over storage types, lengths and places in memory: every row's
- * window fits the chunks that smx_rows_chunks promised, the output window
- * starts on a chunk, and the chosen kernel's waves hold the row. Prints what
+/* The launch rule of the softmax kernels against what their rows really take,
+ * over storage types, lengths and places in memory: every row's window fits
+ * the chunks that smx_rows_chunks promised, the output window starts on a
+ * chunk, the chosen row kernel's waves hold the row, split rows have enough
+ * slices, and a row sent to the "_long_rows" kernels has, by its own chunks,
+ * as many per thread as they rely on and no more than they hold. Prints what
  * does not hold; the exit status is the number of such cases (at most 99). */
 #include <stdio.h>
 #include <stdint.h>
 
 #include "kernel_geometry.h"
+
+/* every length up to 700 and around those where a row takes another kernel
+ * (the sweep stops at each range's start), about every 2000th between */
+static int next_length(int n) {
+	static const int edges[] = {16300, 24500, 32700, 57300, 65400, 98200, 130900, 163700};
+	const int width = 250, n_edges = (int) (sizeof(edges) / sizeof(edges[0]));
+	if (n < 700) return n + 1;
+	for (int i = 0; i < n_edges; i++) {
+		if (n >= edges[i] && n < edges[i] + width) return n + 1;
+		if (n < edges[i] && n + 1997 > edges[i]) return edges[i];
+	}
+	return n + 1997;
+}
 
 int main(void) {
 	static const unsigned long long offsets[] = {0, 16, 64, 112, 2, 6, 34, 128, 4, 12, 8, 1, 5};
@@ -19,7 +34,7 @@ int main(void) {
 		for (int i = 0; i < n_off * n_off; i++) {
 			const unsigned long long x = 4096 + offsets[i / n_off], o = 8192 + offsets[i % n_off];
 			if (x % e || o % oe) continue;
-			for (int n = 1; n < 540000; n += (n < 700 || (n > 130900 && n < 131100)) ? 1 : 1997) {
+			for (int n = 1; n < 540000; n = next_length(n)) {
 				const int bound = smx_rows_chunks(n, e, x, o);
 				if (!bound) continue;
 				const unsigned line = smx_rows_line(n, e, x, o);
@@ -38,6 +53,12 @@ int main(void) {
 						const int per = (sets + s - 1) / s;
 						if (row_counts[k] > SMX_SPLIT_ROWS || s < 1 || s > SMX_SPLIT_MAX || per > SMX_SPLIT_K || (long) s * per * SMX_THREADS < bound) {
 							if (bad++ < 10) printf("elem %d, %d rows of %d columns: %d slices of %d sets\n", e, row_counts[k], n, s, per);
+						}
+					}
+					if (kernel == SMX_LONG_ROWS) {
+						const long nv = (long) n * e / 16, nch = (nv + SMX_THREADS - 1) / SMX_THREADS;
+						if (e != 2 || ((x | o) & 15) || (long) n * e % 16 || nch < smx_regs_atleast(e, SMX_LONG_MAXCH) || nch > SMX_LONG_MAXCH) {
+							if (bad++ < 10) printf("elem %d, %d long rows of %d columns, x+%llu out+%llu: %ld chunks per thread\n", e, row_counts[k], n, x - 4096, o - 8192, nch);
 						}
 					}
 					if (kernel != SMX_ROWS && kernel != SMX_WIDE_ROWS) continue;

@@ -792,6 +792,35 @@ def test_softmax_rows_of_any_alignment(hdl, dt, shape):
         check_f32(d.get(pmean, (1,), np.float32), mean, rel=1e-4, what="fused mean loss")
 
 
+@pytest.mark.parametrize("dt", DTS, ids=dt_id)
+@pytest.mark.parametrize("shape", [(66, 131024, 0), (66, 131064, 0), (66, 131072, 8), (66, 131080, 0), (66, 163840, 8), (66, 163848, 0)],
+                         ids=lambda s: "%dx%d+%d" % s)
+def test_softmax_rows_below_zero_at_16_and_20_chunks(hdl, dt, shape):
+    """Aligned 16-bit rows around 16 and 20 chunks per thread, where the window
+    of whole lines can hold a chunk set more than the row itself, with every
+    logit near -20: a lane past the row's end that counted as a logit of 0
+    would outweigh the whole row by e^20 / n_cols."""
+    from dataflow_lib_amd import api
+    n_rows, n_cols, off = shape
+    es = 4 if dt == FP32 else 2
+    X = to_storage(normal(165, (n_rows, n_cols)) - 20.0, dt)
+    labels = rng(166).integers(0, n_cols, size=n_rows).astype(np.uint32)
+    labels[0], labels[-1] = 0, n_cols - 1
+    pre, lo, hi = (np.empty((n_rows, n_cols)) for _ in range(3))
+    loss, mean = np.empty(n_rows), np.zeros(1)
+    assert oracle().oracle_softmax(dt, dt, n_rows, n_cols, ptr(X), ptr(pre)) == 0
+    assert oracle().oracle_softmax_cross_entropy(dt, n_rows, n_cols, ptr(X), ptr(labels), ptr(lo), ptr(hi), ptr(loss), ptr(mean)) == 0
+    with Dev(hdl) as d:
+        px, po = d.put(X, off * es), d.put(np.zeros_like(X), off * es)
+        assert api.submit_softmax(hdl, 0, dt, dt, n_rows, n_cols, px, po) == 0
+        check_rounded(d.get(po, X.shape, NP_STORAGE[dt]), dt, pre, what="softmax")
+        pl, ploss, pmean = d.put(labels), d.empty(4 * n_rows), d.empty(4)
+        assert api.submit_softmax_cross_entropy_loss(hdl, 0, dt, n_rows, n_cols, px, pl, ploss, pmean) == 0
+        check_rounded(d.get(px, X.shape, NP_STORAGE[dt]), dt, lo, hi, what="fused dlogits")
+        check_f32(d.get(ploss, (n_rows,), np.float32), loss, rel=1e-4, what="fused loss")
+        check_f32(d.get(pmean, (1,), np.float32), mean, rel=1e-4, what="fused mean loss")
+
+
 def test_split_softmax_from_two_threads(hdl):
     """A few long rows take two launches that share the code object's memory:
     submits of two threads on one stream must not come between them. Every
