@@ -268,6 +268,9 @@ GEOM_FN int smx_split_slices(int n_rows, int sets) {
  *   hold in registers (1024 x 128257 bf16 557 us, wide 116);
  * - unaligned rows of more than 16 chunks per thread to SMX_ANY_ROWS, which
  *   streams them as the main kernel does aligned ones;
+ * - rows that would make a launch of the row kernels, which take all rows at
+ *   once, 2^32 threads or more (from 2^26 rows of one wave on), to the main
+ *   kernel, which walks them;
  * - fp8 logits the same way: 12 waves of 8 chunks still share a CU with
  *   another row (1024 x 48000 27.7 us, wide 30.3; 1024 x 50256 43.0, wide
  *   31.6), and the main kernel overlaps rows from some 512 on (300 x 128256
@@ -294,6 +297,8 @@ GEOM_FN int smx_kernel_for(int n_rows, int n_cols, int elem_bytes, unsigned long
 	if (main_regs && elem_bytes == 2 && own > 1024 * SMX_MAXCH && own <= 1024 * SMX_LONG_MAXCH) return SMX_LONG_ROWS;
 	if (chunks == 0) return SMX_MAIN;
 	if (chunks > 1024 * SMX_WIDE_ROWS_CH) return (main_regs || elem_bytes == 1) ? SMX_MAIN : SMX_ANY_ROWS;
+	const int waves = (chunks + 64 * SMX_ROWS_CH - 1) / (64 * SMX_ROWS_CH);   /* at most: the wide kernel takes half */
+	if (64ll * waves * ((long long) n_rows + SMX_ROWS_PER_WG - 1) >= 1ll << 32) return SMX_MAIN;
 	if (elem_bytes == 1) {
 		if (chunks <= (few ? 1024 : 768) * SMX_ROWS_CH) return SMX_ROWS;
 		return (chunks <= 1024 * SMX_ROWS_CH || n_rows <= 2 * SMX_FEW_ROWS || !f8_smx_pf_ok(n_cols)) ? SMX_WIDE_ROWS : SMX_MAIN;

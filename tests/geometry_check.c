@@ -25,7 +25,8 @@ static int next_length(int n) {
 
 int main(void) {
 	static const unsigned long long offsets[] = {0, 16, 64, 112, 2, 6, 34, 128, 4, 12, 8, 1, 5};
-	static const int row_counts[] = {1, 7, 64, 200, 257, 5000};
+	static const int row_counts[] = {1, 7, 64, 200, 257, 5000, 1 << 25, (1 << 26) - 4, 1 << 26, 2147483647};
+	const int n_counts = (int) (sizeof(row_counts) / sizeof(row_counts[0]));
 	const int n_off = (int) (sizeof(offsets) / sizeof(offsets[0]));
 	long bad = 0;
 	for (int e = 1; e <= 4; e *= 2) {
@@ -46,7 +47,7 @@ int main(void) {
 						if (bad++ < 10) printf("elem %d, %d columns, x+%llu out+%llu, row %d: %ld chunks of %d, out %llu\n", e, n, x - 4096, o - 8192, r, need, bound, out & 15);
 					}
 				}
-				for (int k = 0; k < 6; k++) {
+				for (int k = 0; k < n_counts; k++) {
 					const int kernel = smx_kernel_for(row_counts[k], n, e, x, o);
 					if (kernel == SMX_SPLIT) {
 						const int sets = smx_split_sets(n, e, x, o), s = smx_split_slices(row_counts[k], sets);
@@ -66,6 +67,11 @@ int main(void) {
 					const int g = smx_rows_waves(ch, row_counts[k], n, e, x, o);
 					if (g < 1 || g > 16 || (long) g * 64 * ch < bound) {
 						if (bad++ < 10) printf("elem %d, %d rows of %d columns: %d waves of %d chunks for %d\n", e, row_counts[k], n, g, ch, bound);
+					}
+					/* all rows in one launch, whose threads fit 32 bits */
+					const long long threads = g == 1 ? ((long long) row_counts[k] + SMX_ROWS_PER_WG - 1) / SMX_ROWS_PER_WG * 64 * SMX_ROWS_PER_WG : (long long) row_counts[k] * 64 * g;
+					if (threads >= 1ll << 32) {
+						if (bad++ < 10) printf("elem %d, %d rows of %d columns: a launch of %lld threads\n", e, row_counts[k], n, threads);
 					}
 				}
 			}

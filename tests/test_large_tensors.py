@@ -10,7 +10,7 @@ buffer range, lands on different data and fails the comparison."""
 import numpy as np
 import pytest
 
-from support import (BF16, NP_STORAGE, check_f32, check_rounded, gamma, normal, oracle, ptr, rms_ws_depth, rng,
+from support import (BF16, FP8E4M3, FP32, NP_STORAGE, check_f32, check_rounded, gamma, normal, oracle, ptr, rms_ws_depth, rng,
                      to_storage)
 
 pytestmark = pytest.mark.gpu
@@ -133,6 +133,43 @@ def test_fused_cross_entropy_past_4gib(hdl):
     check_rounded(out[:B], dt, lo, hi, what="fused dlogits")
     assert_blocks_equal(out, B, "fused dlogits")
     del out
+    check_f32(gl[:B], loss, rel=1e-4, what="fused loss")
+    assert_blocks_equal(gl, B, "fused loss")
+    check_f32(gm, mean, rel=1e-4, what="fused mean loss")
+
+
+@pytest.mark.parametrize("case", [(BF16, BF16, 2), (BF16, BF16, 8), (FP32, FP32, 1), (FP8E4M3, BF16, 2)],
+                         ids=["bf16x2", "bf16x8", "fp32x1", "e4m3x2"])
+def test_softmax_past_2_26_rows(hdl, case):
+    """67,108,867 rows of a few columns, seven distinct ones repeated: 64
+    threads a row, as the kernels for short rows launch them, would be past
+    2^32 threads, which one launch cannot have, so the main kernel walks them."""
+    from dataflow_lib_amd import api
+    dt, odt, C = case
+    B, reps = 7, 9586981
+    R = B * reps
+    assert 64 * R > 1 << 32
+    X = to_storage(normal(215, (B, C), std=2.0), dt)
+    lab = (np.arange(B) % C).astype(np.uint32)
+    pre = np.empty((B, C))
+    assert oracle().oracle_softmax(dt, odt, B, C, ptr(X), ptr(pre)) == 0
+    with Bufs(hdl) as d:
+        px, po = d.tiled(X, reps), d.empty(R * C * NP_STORAGE[odt]().itemsize)
+        assert api.submit_softmax(hdl, 0, dt, odt, R, C, px, po) == 0
+        out = d.get(po, (R, C), NP_STORAGE[odt])
+        check_rounded(out[:B], odt, pre, what="softmax")
+        assert_blocks_equal(out, B, "softmax")
+        del out
+        if dt == FP8E4M3:   # the fused loss has no fp8 form
+            return
+        lo, hi, loss, mean = np.empty((B, C)), np.empty((B, C)), np.empty(B), np.zeros(1)
+        assert oracle().oracle_softmax_cross_entropy(dt, B, C, ptr(X), ptr(lab), ptr(lo), ptr(hi), ptr(loss), ptr(mean)) == 0
+        pl, ploss, pmean = d.tiled(lab, reps), d.empty(4 * R), d.empty(4)
+        assert api.submit_softmax_cross_entropy_loss(hdl, 0, dt, R, C, px, pl, ploss, pmean) == 0
+        gl, gm = d.get(ploss, (R,), np.float32), d.get(pmean, (1,), np.float32)
+        out = d.get(px, (R, C), NP_STORAGE[dt])
+    check_rounded(out[:B], dt, lo, hi, what="fused dlogits")
+    assert_blocks_equal(out, B, "fused dlogits")
     check_f32(gl[:B], loss, rel=1e-4, what="fused loss")
     assert_blocks_equal(gl, B, "fused loss")
     check_f32(gm, mean, rel=1e-4, what="fused mean loss")
