@@ -701,7 +701,8 @@ __device__ __forceinline__ SmxWindow smx_window(const T * X, TO * out, int n_col
 	return w;
 }
 
-/* any row length / alignment: three passes over global memory per row */
+/* any row length / alignment: three passes over global memory per row (the
+ * column index is unsigned: a step past 2^31 - 1 columns does not wrap) */
 template <typename T, typename TO, bool FUSED>
 __device__ __forceinline__ void smx_stream(int n_rows, int n_cols, const T * X, TO * out, const uint32_t * labels, float * loss) {
 	__shared__ float slots[32];
@@ -717,20 +718,20 @@ __device__ __forceinline__ void smx_stream(int n_rows, int n_cols, const T * X, 
 			if (tid == 0 && lab < (uint32_t) n_cols) x_lab = to_f(xrow[lab]);
 		}
 		float m = -__builtin_inff();
-		for (int j = tid; j < n_cols; j += nt) m = fmaxf(m, to_f(xrow[j]));
+		for (uint32_t j = tid; j < (uint32_t) n_cols; j += nt) m = fmaxf(m, to_f(xrow[j]));
 		m = block_max(m, slots);
 		float sd = 0.0f, sx = 0.0f;
-		for (int j = tid; j < n_cols; j += nt) {
+		for (uint32_t j = tid; j < (uint32_t) n_cols; j += nt) {
 			const float diff = to_f(xrow[j]) - m;
 			sd += exp_fast(rnd_in<T>(diff));
-			if (FUSED && (uint32_t) j != lab) sx += exp_fast(diff);
+			if (FUSED && j != lab) sx += exp_fast(diff);
 		}
 		__syncthreads();
 		block_sum2(sd, sx, slots);
 		const float inv = 1.0f / sd;
-		for (int j = tid; j < n_cols; j += nt) {
+		for (uint32_t j = tid; j < (uint32_t) n_cols; j += nt) {
 			float y = exp_fast(rnd_in<T>(to_f(xrow[j]) - m)) * inv;
-			if (FUSED && (uint32_t) j == lab) y = rnd_in<TO>(y) - 1.0f;
+			if (FUSED && j == lab) y = rnd_in<TO>(y) - 1.0f;
 			orow[j] = from_f<TO>(y);
 		}
 		if (FUSED && tid == 0 && loss) {

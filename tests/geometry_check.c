@@ -77,5 +77,20 @@ int main(void) {
 			}
 		}
 	}
+	/* rows of gigabytes: the "_any_rows" kernels' byte offsets and element
+	 * indexes, which run up to four sets of chunks past the row, in 32 bits */
+	static const int huge[] = {1 << 28, (1 << 29) + 3, (1 << 30) - 32769, (1 << 30) - 1, 1 << 30, (1 << 30) + 5, 2147483647 - 65600, 2147483647 - 64, 2147483647};
+	for (int i = 0; i < (int) (sizeof(huge) / sizeof(huge[0])); i++) {
+		for (int e = 2; e <= 4; e *= 2) {
+			for (unsigned long long off = 0; off < 128; off += e) {
+				const int n = huge[i];
+				if (smx_kernel_for(1, n, e, 4096 + off, 8192 + off) != SMX_ANY_ROWS) continue;
+				const long long last = ((long long) n * e + 127) / 16 + 1 + 4 * SMX_THREADS;
+				if (last * 16 >= 1ll << 32 || last * (16 / e) >= 1ll << 31) {
+					if (bad++ < 10) printf("elem %d, a row of %d columns +%llu: byte %lld, element %lld\n", e, n, off, last * 16, last * (16 / e));
+				}
+			}
+		}
+	}
 	return bad > 99 ? 99 : (int) bad;
 }

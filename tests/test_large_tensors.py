@@ -175,6 +175,26 @@ def test_softmax_past_2_26_rows(hdl, case):
     check_f32(gm, mean, rel=1e-4, what="fused mean loss")
 
 
+def test_softmax_row_past_4gib(hdl):
+    """One fp32 row of 8193 copies of 131071 columns (4.3 GB), which is not a
+    multiple of 16 bytes: every copy's outputs equal the first's bit for bit,
+    and those a copy's softmax / 8193 up to the sum's roundings (a thread's
+    columns in sequence, the waves' tree)."""
+    from dataflow_lib_amd import api
+    L, reps = 131071, 8193
+    n = L * reps
+    assert 4 * n > FOUR_GIB and n % 4 != 0
+    X = normal(217, (1, L), std=2.0)
+    pre = np.empty((1, L))
+    assert oracle().oracle_softmax(FP32, FP32, 1, L, ptr(X), ptr(pre)) == 0
+    with Bufs(hdl) as d:
+        px, po = d.tiled(X, reps), d.empty(4 * n)
+        assert api.submit_softmax(hdl, 0, FP32, FP32, 1, n, px, po) == 0
+        out = d.get(po, (reps, L), np.float32)
+    check_f32(out[0], pre / reps, rel=gamma(-(-n // 1024) + 6 + 16) + 1e-5, what="softmax of a long row")
+    assert_blocks_equal(out, 1, "softmax of a long row")
+
+
 def test_rms_norm_past_4gib(hdl):
     """fwd and bwd_x over 524293 x 4096 bf16 rows (4.3 GB per tensor), seven
     distinct rows repeated; 2^32 bytes is exactly 524288 rows, which is not a
