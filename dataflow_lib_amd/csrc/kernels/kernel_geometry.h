@@ -242,6 +242,10 @@ GEOM_FN int smx_split_slices(int n_rows, int sets) {
 	return (sets + k - 1) / k;
 }
 
+/* streaming kernels: rows of 2^28 chunks (4 GiB), which 32-bit offsets do not
+ * reach, less more than the four sets of chunks that a pass runs past the row */
+#define SMX_STREAM_MAX_CHUNKS ((1 << 28) - (1 << 13))
+
 /* Which kernel a softmax / cross-entropy call takes. In order:
  * - SMX_SPLIT for at most SMX_SPLIT_ROWS rows (half as many of 8 sets) of more
  *   than seven (fp32: eight) sets of SMX_THREADS chunks, in slices of at most
@@ -267,9 +271,9 @@ GEOM_FN int smx_split_slices(int n_rows, int sets) {
  *   fp32 169.4, wide 184.1), unless they are unaligned, which it does not
  *   hold in registers (1024 x 128257 bf16 557 us, wide 116);
  * - unaligned rows of more than 16 chunks per thread to SMX_ANY_ROWS, which
- *   streams them as the main kernel does aligned ones, with 32-bit offsets:
- *   rows of SMX_ANY_MAX_CHUNKS chunks (4 GiB) and more go element by element
- *   in the main kernel;
+ *   streams them as the main kernel does aligned ones, but for rows of
+ *   SMX_STREAM_MAX_CHUNKS chunks and more, which go element by element in the
+ *   main kernel;
  * - rows that would make a launch of the row kernels, which take all rows at
  *   once, 2^32 threads or more (from 2^26 rows of one wave on), to the main
  *   kernel, which walks them;
@@ -284,8 +288,6 @@ GEOM_FN int smx_split_slices(int n_rows, int sets) {
 #define SMX_LONG_ROWS 3
 #define SMX_SPLIT 4
 #define SMX_ANY_ROWS 5
-/* less what a pass runs past the row: four sets of SMX_THREADS chunks */
-#define SMX_ANY_MAX_CHUNKS ((1 << 28) - (1 << 13))
 #define SMX_FEW_ROWS 256   /* no more rows than CUs: each row has a CU to itself */
 GEOM_FN int smx_kernel_for(int n_rows, int n_cols, int elem_bytes, unsigned long long x, unsigned long long out) {
 	const int chunks = smx_rows_chunks(n_cols, elem_bytes, x, out);
@@ -300,7 +302,7 @@ GEOM_FN int smx_kernel_for(int n_rows, int n_cols, int elem_bytes, unsigned long
 	const long own = (long) n_cols * elem_bytes / 16;
 	if (main_regs && elem_bytes == 2 && own > 1024 * SMX_MAXCH && own <= 1024 * SMX_LONG_MAXCH) return SMX_LONG_ROWS;
 	if (chunks == 0) return SMX_MAIN;
-	if (chunks > 1024 * SMX_WIDE_ROWS_CH) return (main_regs || elem_bytes == 1 || chunks >= SMX_ANY_MAX_CHUNKS) ? SMX_MAIN : SMX_ANY_ROWS;
+	if (chunks > 1024 * SMX_WIDE_ROWS_CH) return (main_regs || elem_bytes == 1 || chunks >= SMX_STREAM_MAX_CHUNKS) ? SMX_MAIN : SMX_ANY_ROWS;
 	const int waves = (chunks + 64 * SMX_ROWS_CH - 1) / (64 * SMX_ROWS_CH);   /* at most: the wide kernel takes half */
 	if (64ll * waves * ((long long) n_rows + SMX_ROWS_PER_WG - 1) >= 1ll << 32) return SMX_MAIN;
 	if (elem_bytes == 1) {

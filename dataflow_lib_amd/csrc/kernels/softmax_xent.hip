@@ -975,7 +975,8 @@ __device__ __forceinline__ void smx(int n_rows, int n_cols, const T * X, TO * ou
 						&& ((n_cols / VEC + SMX_THREADS - 1) / SMX_THREADS) <= SMX_MAXCH
 						&& ((n_cols / VEC + SMX_THREADS - 1) / SMX_THREADS) >= smx_regs_atleast((int) sizeof(T), SMX_MAXCH);
 	if (vec_ok) smx_regs<T, TO, FUSED>(n_rows, n_cols, X, out, labels, loss);
-	else if (sizeof(TO) == sizeof(T) && n_cols % VEC == 0 && aligned16(X) && aligned16(out) && blockDim.x == SMX_THREADS)
+	else if (sizeof(TO) == sizeof(T) && n_cols % VEC == 0 && n_cols / VEC < SMX_STREAM_MAX_CHUNKS && aligned16(X) && aligned16(out) &&
+			 blockDim.x == SMX_THREADS)
 		smx_stream_vec<T, FUSED>(n_rows, n_cols, X, reinterpret_cast<T *>(out), labels, loss);
 	else smx_stream<T, TO, FUSED>(n_rows, n_cols, X, out, labels, loss);
 	smx_launch_end<FUSED>(n_rows, loss, mean_loss);

@@ -175,15 +175,16 @@ def test_softmax_past_2_26_rows(hdl, case):
     check_f32(gm, mean, rel=1e-4, what="fused mean loss")
 
 
-def test_softmax_row_past_4gib(hdl):
-    """One fp32 row of 8193 copies of 131071 columns (4.3 GB), which is not a
-    multiple of 16 bytes: every copy's outputs equal the first's bit for bit,
+@pytest.mark.parametrize("L", [131071, 131072])
+def test_softmax_row_past_4gib(hdl, L):
+    """One fp32 row of 8193 copies of L columns (4.3 GB; odd, so not a multiple
+    of 16 bytes, and aligned): every copy's outputs equal the first's bit for bit,
     and those a copy's softmax / 8193 up to the sum's roundings (a thread's
     columns in sequence, the waves' tree)."""
     from dataflow_lib_amd import api
-    L, reps = 131071, 8193
+    reps = 8193
     n = L * reps
-    assert 4 * n > FOUR_GIB and n % 4 != 0
+    assert 4 * n > FOUR_GIB
     X = normal(217, (1, L), std=2.0)
     pre = np.empty((1, L))
     assert oracle().oracle_softmax(FP32, FP32, 1, L, ptr(X), ptr(pre)) == 0
