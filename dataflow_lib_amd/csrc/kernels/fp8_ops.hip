@@ -372,9 +372,11 @@ __device__ __forceinline__ void softmax_fp8_pf(int n_rows, int n_cols, const TF 
 	vmem_wait_all();
 }
 
-/* Other rows (of more than 131,072 columns, or unaligned tensors): three passes per row, the later ones re-reading the row (a
- * row of fp8 is n_cols bytes, so they find it in cache): max, sum exp(d),
- * outputs. In both paths d = rnd_out(x - max), since the reference converts x
+/* Other rows (of more than 131,072 columns, unaligned tensors, or 2^26 rows
+ * and more): three passes per row, the later ones re-reading the row (a row
+ * of fp8 is n_cols bytes, so they find it in cache): max, sum exp(d), outputs.
+ * Row and column indexes are unsigned, so that a step past 2^31 - 1 does not
+ * wrap. In both paths d = rnd_out(x - max), since the reference converts x
  * to the output type and subtracts there. */
 template <typename TF, typename TO>
 __device__ __forceinline__ void softmax_fp8(int n_rows, int n_cols, const TF * X, TO * out) {
@@ -386,7 +388,7 @@ __device__ __forceinline__ void softmax_fp8(int n_rows, int n_cols, const TF * X
 	}
 	const bool vec = (n_cols % 8) == 0 && aligned8(X) && aligned16(out);
 	const int nv = n_cols / 8;
-	for (int row = blockIdx.x; row < n_rows; row += gridDim.x) {
+	for (uint32_t row = blockIdx.x; row < (uint32_t) n_rows; row += gridDim.x) {
 		const TF * x = X + (long) row * n_cols;
 		TO * o = out + (long) row * n_cols;
 		float m = -__builtin_inff();
@@ -399,7 +401,7 @@ __device__ __forceinline__ void softmax_fp8(int n_rows, int n_cols, const TF * X
 			}
 		}
 		else {
-			for (int j = threadIdx.x; j < n_cols; j += blockDim.x) m = __builtin_elementwise_maximum(m, to_f(x[j]));
+			for (uint32_t j = threadIdx.x; j < (uint32_t) n_cols; j += blockDim.x) m = __builtin_elementwise_maximum(m, to_f(x[j]));
 		}
 		m = block_max(m, slots);
 		float sd = 0.0f;
@@ -412,7 +414,7 @@ __device__ __forceinline__ void softmax_fp8(int n_rows, int n_cols, const TF * X
 			}
 		}
 		else {
-			for (int j = threadIdx.x; j < n_cols; j += blockDim.x) sd += exp_fast(rnd_in<TO>(to_f(x[j]) - m));
+			for (uint32_t j = threadIdx.x; j < (uint32_t) n_cols; j += blockDim.x) sd += exp_fast(rnd_in<TO>(to_f(x[j]) - m));
 		}
 		float unused = 0.0f;
 		__syncthreads();   /* every wave has read the max cells */
@@ -428,7 +430,7 @@ __device__ __forceinline__ void softmax_fp8(int n_rows, int n_cols, const TF * X
 			}
 		}
 		else {
-			for (int j = threadIdx.x; j < n_cols; j += blockDim.x)
+			for (uint32_t j = threadIdx.x; j < (uint32_t) n_cols; j += blockDim.x)
 				o[j] = from_f<TO>(__builtin_amdgcn_exp2f(fmaf(rnd_in<TO>(to_f(x[j]) - m), SMX_LOG2E, nlog2s)));
 		}
 		__syncthreads();   /* the cells are rewritten for the next row */

@@ -200,7 +200,7 @@ __device__ __forceinline__ void smx_launch_end(int n_rows, const float * loss, f
 	if (FUSED && loss && mean_loss) {
 		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 		double s = 0.0;
-		for (int r = threadIdx.x; r < n_rows; r += blockDim.x) s += (double) __hip_atomic_load(loss + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		for (uint32_t r = threadIdx.x; r < (uint32_t) n_rows; r += blockDim.x) s += (double) __hip_atomic_load(loss + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
 		if ((threadIdx.x & 63) == 0) dslots[threadIdx.x >> 6] = s;
 		__syncthreads();
@@ -702,13 +702,13 @@ __device__ __forceinline__ SmxWindow smx_window(const T * X, TO * out, int n_col
 }
 
 /* any row length / alignment: three passes over global memory per row (the
- * column index is unsigned: a step past 2^31 - 1 columns does not wrap) */
+ * row and column indexes are unsigned: a step past 2^31 - 1 does not wrap) */
 template <typename T, typename TO, bool FUSED>
 __device__ __forceinline__ void smx_stream(int n_rows, int n_cols, const T * X, TO * out, const uint32_t * labels, float * loss) {
 	__shared__ float slots[32];
 	const int tid = threadIdx.x;
 	const int nt = blockDim.x;
-	for (int row = blockIdx.x; row < n_rows; row += gridDim.x) {
+	for (uint32_t row = blockIdx.x; row < (uint32_t) n_rows; row += gridDim.x) {
 		const T * xrow = X + (long) row * n_cols;
 		TO * orow = out + (long) row * n_cols;
 		uint32_t lab = 0xffffffffu;

@@ -196,6 +196,26 @@ def test_softmax_row_past_4gib(hdl, L):
     assert_blocks_equal(out, 1, "softmax of a long row")
 
 
+def test_softmax_fp8_row_of_2_31_columns(hdl):
+    """One row of 2^31 - 2 e4m3 logits, 65538 copies of 32767: a column index
+    that steps by the workgroup's 1024 threads passes 2^31. The tolerance is
+    the sum's roundings (a thread's columns in sequence, the waves') and the
+    output's ulp."""
+    from dataflow_lib_amd import api
+    L, reps = 32767, 65538
+    n = L * reps
+    assert n < (1 << 31) and n + 1024 > 1 << 31
+    X = to_storage(normal(218, (1, L), std=2.0), FP8E4M3)
+    pre = np.empty((1, L))
+    assert oracle().oracle_softmax(FP8E4M3, BF16, 1, L, ptr(X), ptr(pre)) == 0
+    with Bufs(hdl) as d:
+        px, po = d.tiled(X, reps), d.empty(2 * n)
+        assert api.submit_softmax(hdl, 0, FP8E4M3, BF16, 1, n, px, po) == 0
+        out = d.get(po, (reps, L), NP_STORAGE[BF16])
+    check_rounded(out[0], BF16, pre / reps, floor=gamma(-(-n // 1024) + 6 + 16) * pre / reps, what="softmax of a long fp8 row")
+    assert_blocks_equal(out, 1, "softmax of a long fp8 row")
+
+
 def test_rms_norm_past_4gib(hdl):
     """fwd and bwd_x over 524293 x 4096 bf16 rows (4.3 GB per tensor), seven
     distinct rows repeated; 2^32 bytes is exactly 524288 rows, which is not a
