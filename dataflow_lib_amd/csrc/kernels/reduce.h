@@ -23,6 +23,14 @@ __device__ __forceinline__ void lds_barrier() {
 	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+/* orders this wave's LDS writes and reads among its lanes (LDS only, so the
+ * wave's global loads and stores stay in flight) */
+__device__ __forceinline__ void wave_lds_sync() {
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float v) {
 	return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));

@@ -38,14 +38,6 @@ __device__ __forceinline__ void rotate(float c, float s, float e, float o, float
 	}
 }
 
-/* orders this wave's LDS table writes and reads (LDS only, so the wave's
- * global loads and stores stay in flight) */
-__device__ __forceinline__ void wave_lds_sync() {
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 /* rotate one row (Q or K) of `width` elements with the token's table; the
  * rotated row is also written to `mirror` when it is not null (16-byte
  * aligned on the vector path) */

@@ -330,6 +330,7 @@ __device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, TO
 	float sd = sd0 + sd1;
 	waves_sum2(sd, sx, scells, g, wave, lane);
 	if (FUSED && wave == 0 && loss) {
+		if (g == 1) wave_lds_sync();   /* the labelled logit, another lane's (g > 1: the sums' barrier) */
 		if (lane == 0) store_loss(loss, row, lab_ok ? fused_loss(sx, m, xlab_cell[cell]) : __builtin_nanf(""));
 		/* a workgroup of one row counts it before the outputs, so that the
 		 * store, the count and the sums that follow it run beside them */
