@@ -10,6 +10,19 @@
 
 #include "kernel_geometry.h"
 
+/* Which kernel, and which of the main kernels' paths (as they choose it), a
+ * softmax call takes: an index into ROUTES of test_geometry.py. */
+int smx_route(int n_rows, int n_cols, int elem, unsigned long long x, unsigned long long out) {
+	const int kernel = smx_kernel_for(n_rows, n_cols, elem, x, out);
+	if (kernel != SMX_MAIN) return kernel;
+	const int aligned = ((x | out) & 15) == 0;
+	if (elem == 1) return aligned && f8_smx_pf_ok(n_cols) ? SMX_MAIN : 7;
+	const long nv = (long) n_cols * elem / 16, nch = (nv + SMX_THREADS - 1) / SMX_THREADS;
+	if (!aligned || (long) n_cols * elem % 16 != 0) return 7;
+	if (nch <= SMX_MAXCH && nch >= smx_regs_atleast(elem, SMX_MAXCH)) return SMX_MAIN;
+	return nv < SMX_STREAM_MAX_CHUNKS ? 6 : 7;
+}
+
 /* every length up to 700 and around those where a row takes another kernel
  * (the sweep stops at each range's start), about every 2000th between */
 static int next_length(int n) {

@@ -320,18 +320,20 @@ def test_swiglu_bwd_fp8(hdl, fb, shape):
 
 # ---------------- softmax ----------------
 
-# rows of 32768..131072 columns (a multiple of 16) take the path that prefetches
-# the next row: (300, 32768), (520, 65552), (260, 128256) and (1100, 128256)
-# give workgroups several rows each (more rows than CUs; four or five in the
-# last), 65552 leaves two 8-byte pieces in the register half, (2, 131072) is
-# the longest such row
+# more than 512 rows of 65,544 to 131,072 columns (a multiple of 16) take the
+# path that prefetches the next row: (520, 65552), which leaves two 8-byte
+# pieces in the register half, (1100, 128256) and (520, 131072), the longest
+# such rows; fewer rows are held by 16 chunks per thread ((260, 128256)), up to
+# 64 split over workgroups ((4, 128256), (2, 131072)), shorter ones held by 1
+# to 16 waves
 SMX_SHAPES = [(4, 128256), (3, 1000), (2, 1001), (2, 140000), (5, 64), (1, 1), (7, 4104),
               (300, 32768), (520, 65552), (260, 128256), (2, 131072), (5, 65536), (1100, 128256)]
 # rows of one wave, of several, and of 16 chunks per thread, whose 8-byte
 # chunks reach into the rows beside them; many short rows
 SMX_SHAPES += [(9, 513), (5, 4097), (300, 16383), (3, 49161), (300, 49145), (2, 65529), (2, 130001), (3, 131064), (600, 33), (64, 60000), (70, 100001)]
-# logits placed off 16-byte alignment: the element-wise loop (for (5, 65536),
-# with the long-row path's workgroup size)
+# the prefetching path's longest rows, and longer ones, read three times
+SMX_SHAPES += [(520, 131072), (70, 140000)]
+# logits placed off 16-byte alignment: the element-wise loop
 SMX_UNALIGNED = ((2, 1001), (5, 65536))
 
 
@@ -358,12 +360,17 @@ def test_softmax_fp8(hdl, fb, shape):
     assert np.allclose(to_f64(out, bdt).sum(axis=1), 1.0, atol=2e-2)
 
 
+SMX_SPECIAL = [(300, 32768), (600, 4104), (600, 65552), (300, 100001), (8, 100000), (70, 140000)]
+
+
 @pytest.mark.parametrize("fb", MIXED, ids=MIXED_IDS)
-@pytest.mark.parametrize("shape", [(300, 32768), (600, 4104)], ids=lambda s: "%dx%d" % s)
+@pytest.mark.parametrize("shape", SMX_SPECIAL, ids=lambda s: "%dx%d" % s)
 def test_softmax_fp8_special_rows(hdl, fb, shape):
-    """workgroups walking several rows (the prefetching path and the
-    two-workgroup path) through an all -inf row, a row with +inf and one with
-    NaN (E4M3 has no infinities: they saturate to -448 / 448)"""
+    """An all -inf row, a row with +inf and one with NaN (E4M3 has no
+    infinities: they saturate to -448 / 448) on every kernel: 8 chunks per
+    thread (300 x 32768, 600 x 4104), workgroups walking several prefetched
+    rows (600 x 65552), 16 chunks per thread (300 x 100001), split rows
+    (8 x 100000) and rows read three times (70 x 140000)"""
     from dataflow_lib_amd import api
     fdt, bdt = fb
     n_rows, n_cols = shape
@@ -383,17 +390,19 @@ def test_softmax_fp8_special_rows(hdl, fb, shape):
     assert np.isnan(to_f64(out, bdt)[n_rows - 3]).all()
 
 
-def test_softmax_fp8_on_two_streams_matches_one_stream(hdl):
+@pytest.mark.parametrize("ce_shape", [(600, 32000), (600, 66000)], ids=lambda s: "%dx%d" % s)
+def test_softmax_fp8_on_two_streams_matches_one_stream(hdl, ce_shape):
     """The fp8 softmax's long-row path hands rows out from the same counter in
-    the code object as the 16-bit fused loss op (and counts finished
-    workgroups there), so the handle orders the two across its streams: the
+    the code object as the 16-bit fused loss op on rows held whole (600 x
+    66000; 600 x 32000 counts rows in groups of its own), and counts finished
+    workgroups there, so the handle orders the two across its streams: the
     two ops alternating between streams without waits, with more rows than
     two per workgroup so that both take tickets, give the same bits as the
     same launches on one stream, and the fp8 probabilities match the oracle."""
     from dataflow_lib_amd import api
     from test_hip_ops import logits
     fdt, bdt = FP8E4M3, BF16
-    ce_shape, sm_shape = (600, 32000), (600, 65552)
+    sm_shape = (600, 65552)
     Xc = logits(BF16, ce_shape, seed=160)
     lab = rng(161).integers(0, ce_shape[1], size=ce_shape[0]).astype(np.uint32)
     Xs = to_storage(normal(162, sm_shape, std=2.0), fdt)

@@ -652,15 +652,19 @@ def test_swiglu_unaligned(hdl):
 # ---------------- softmax / cross-entropy ----------------
 
 SMX_SHAPES = [(4, 128256), (3, 1000), (2, 1001), (2, 140000), (5, 64), (1, 1)]
-# rows just past the register path (16-bit: 131,072 columns, fp32: 65,536),
-# where one thread holds one chunk more than the others, and a row of 32
-# (16-bit) or 64 (fp32) chunks per thread, of which the first 6-16 are held
+# few long rows, split over workgroups up to 64 sets of chunks (fp32: the last),
+# with one chunk in their last set
 SMX_SHAPES += [(5, 131080), (4, 65540), (3, 262144)]
+# the same lengths for one workgroup each: just past 16 chunks per thread
+# (16-bit: the 20-chunk kernel, fp32: streamed), 32 (16-bit) or 64 (fp32)
+# chunks per thread, of which the first 6-16 are held, and the Llama-3
+# vocabulary (16-bit: held whole)
+SMX_SHAPES += [(66, 131080), (65, 65540), (65, 262144), (66, 128256)]
 SMX_SHAPES += [(_ri(1, 40), _ri(1, 150000)), (_ri(1, 40), 8 * _ri(1, 16384))]
-# long rows on the streaming path with more rows than workgroups, so rows past
-# each workgroup's first are handed out by ticket (600 x 140,000: every type
-# streams; 16-bit rows of 70,000 stay on the register path)
-SMX_SHAPES += [(600, 140000)]
+# long rows with more rows than workgroups, so that later ones are handed out
+# by ticket: 600 x 140,000 (16-bit: 20 chunks per thread, fp32: streamed),
+# 300 x 200,000 (every type streams) and 560 x 66,000 (16-bit: held whole)
+SMX_SHAPES += [(600, 140000), (300, 200000), (560, 66000)]
 
 
 def logits(dt, shape, seed=101):
@@ -749,7 +753,8 @@ ROW_SHAPES = [(9, 2047, 0), (9, 2049, 1), (5, 4088, 0), (5, 4097, 3), (7, 16385,
               (3, 65544, 8), (2, 131001, 0), (2, 131073, 1), (259, 40001, 0), (2051, 200, 0), (523, 65, 7),
               (17, 57400, 0), (64, 58001, 3), (65, 58000, 0), (1, 200001, 1), (40, 66000, 0),   # few long rows: split over workgroups
               (67, 131201, 0), (65, 163901, 3), (300, 70001, 1),   # unaligned rows past 16 chunks per thread (fp32: the last)
-              (2, 163840, 0), (2, 163848, 0)]   # the last 16-bit row held in 20 chunks per thread, and one past it
+              (2, 163840, 0), (2, 163848, 0),   # split, the last chunk in a set of its own
+              (66, 131080, 0), (66, 163840, 8), (66, 163848, 0)]   # 17 and 20 chunks per thread of 16-bit rows, and one chunk past
 
 
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
@@ -821,6 +826,26 @@ def test_softmax_rows_below_zero_at_16_and_20_chunks(hdl, dt, shape):
         check_f32(d.get(pmean, (1,), np.float32), mean, rel=1e-4, what="fused mean loss")
 
 
+@pytest.mark.parametrize("dt", DTS, ids=dt_id)
+@pytest.mark.parametrize("shape", [(70, 1000), (9, 2049), (66, 128256), (3, 131080)], ids=lambda s: "%dx%d" % s)
+def test_softmax_input_and_output_placed_differently(hdl, dt, shape):
+    """Logits and probabilities that lie differently within 16 bytes: no chunk
+    of the one is a chunk of the other, so the rows go element by element."""
+    from dataflow_lib_amd import api
+    n_rows, n_cols = shape
+    es, pad = (4 if dt == FP32 else 2), 64
+    X = special_logits(dt, shape, seed=167) if n_rows > 4 else logits(dt, shape, seed=167)
+    pre = np.empty(shape)
+    assert oracle().oracle_softmax(dt, dt, n_rows, n_cols, ptr(X), ptr(pre)) == 0
+    guard = np.full(X.size + 2 * pad, 7, X.dtype)
+    with Dev(hdl) as d:
+        px, po = d.put(X), d.put(guard)
+        assert api.submit_softmax(hdl, 0, dt, dt, n_rows, n_cols, px, po + (pad + 1) * es) == 0
+        out = d.get(po, guard.shape, X.dtype)
+    assert (out[:pad + 1] == 7).all() and (out[pad + 1 + X.size:] == 7).all()
+    check_rounded(out[pad + 1:pad + 1 + X.size].reshape(shape), dt, pre, what="softmax")
+
+
 def test_split_softmax_from_two_threads(hdl):
     """A few long rows take two launches that share the code object's memory:
     submits of two threads on one stream must not come between them. Every
@@ -855,15 +880,19 @@ def test_split_softmax_from_two_threads(hdl):
                 assert np.array_equal(d.get(po[k][i], X[k].shape, np.uint16), want), (k, i)
 
 
-# more rows than workgroups (each walks 2-3 rows with the next row, its label
-# and labelled logit in flight); 32000 and 24576 + 8 columns leave a partial
-# last chunk, 128256 is the Llama-3 vocabulary
-MANY_ROWS = [(700, 32000), (600, 24584), (300, 128256), (300, 151936)]   # 151936: half-precision rows past the register path
+# more rows than CUs. 300 rows of 128,256 (16-bit) and 151,936 columns: each
+# workgroup walks one or two with the next row, its label and labelled logit
+# in flight; 32000 and 24576 + 8 columns leave a partial last chunk
+MANY_ROWS = [(700, 32000), (600, 24584), (300, 128256), (300, 151936)]
 MANY_ROWS += [(_ri(257, 700), 8 * _ri(125, 16032))]
+# special rows on every kernel: held whole (16-bit; fp32 70 x 65536), streamed
+# (aligned; fp32 also the ones before), split, streamed unaligned, 16 chunks
+# per thread, short
+SPECIAL_ROWS = [(66, 128256), (70, 65536), (66, 151936), (70, 200000), (8, 128256), (67, 131201), (300, 50257), (600, 1001)]
 
 
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
-@pytest.mark.parametrize("shape", MANY_ROWS, ids=lambda s: "%dx%d" % s)
+@pytest.mark.parametrize("shape", MANY_ROWS + SPECIAL_ROWS, ids=lambda s: "%dx%d" % s)
 def test_softmax_cross_entropy_many_rows(hdl, dt, shape):
     from dataflow_lib_amd import api
     n_rows, n_cols = shape
@@ -888,7 +917,7 @@ def test_softmax_cross_entropy_many_rows(hdl, dt, shape):
 
 
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
-@pytest.mark.parametrize("shape", MANY_ROWS[:2], ids=lambda s: "%dx%d" % s)
+@pytest.mark.parametrize("shape", MANY_ROWS[:2] + SPECIAL_ROWS, ids=lambda s: "%dx%d" % s)
 def test_softmax_many_rows(hdl, dt, shape):
     from dataflow_lib_amd import api
     n_rows, n_cols = shape
@@ -941,9 +970,10 @@ def shifted_logits(dt, shape, seed):
     return to_storage(x, dt)
 
 
-SHIFTED_SHAPES = [(6, 128256), (6, 151936), (6, 1001)]   # register path (16-bit), streaming vector path, element path
-# the same lengths where there are too many rows to split them over workgroups
-WHOLE_ROW_SHAPES = [(66, 128256), (66, 151936)]
+SHIFTED_SHAPES = [(6, 128256), (6, 151936), (6, 1001)]   # split over workgroups, and several waves per row
+# too many rows to split: held whole (16-bit; fp32 66 x 65536), 20 chunks per
+# thread (16-bit), streamed aligned and unaligned
+WHOLE_ROW_SHAPES = [(66, 128256), (66, 151936), (66, 65536), (66, 200000), (67, 131201)]
 
 
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
@@ -969,23 +999,27 @@ def test_fused_loss_on_shifted_rows(hdl, dt, shape):
     check_f32(gm, mean, rel=1e-4, what="fused mean loss, shifted rows")
 
 
+FAR_CASES = [(16, 1.0, -1.0e4), (16, 1.0, 1.0e4), (1000, 10.0, -1.0e4), (1000, 10.0, 1.0e4)]
+FAR_CASES += [(65536, 10.0, -1.0e4), (65536, 10.0, 1.0e4)]
+
+
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
-@pytest.mark.parametrize("case", [(16, 1.0, -1.0e4), (16, 1.0, 1.0e4), (1000, 10.0, -1.0e4), (1000, 10.0, 1.0e4)],
-                         ids=lambda c: "%dcols_std%g_shift%g" % c)
+@pytest.mark.parametrize("case", FAR_CASES, ids=lambda c: "%dcols_std%g_shift%g" % c)
 def test_fused_loss_on_short_rows_far_from_zero(hdl, dt, case):
-    """Short rows of logits near +-1e4 on the register path (600 rows, so
-    workgroups take tickets), the label holding the row max by one step of
+    """Rows of logits near +-1e4, the label holding the row max by one step of
     the storage type there (8 in fp32 and fp16, 64 in bf16), so the losses
     are about the sum of the other columns' exp(x - x_label), small numbers
-    whose relative precision rests on that sum. It is taken against a
-    reference that trails the row max; a rounding of that reference that is
-    not cancelled exactly shows as a relative error up to ~3e-4 at |x| = 1e4
-    (an fp32 ulp of x log2(e)): a form of the kernel that kept the reference
-    in the log2 domain and clamped the final rescale's exponent at 0 failed
-    here on about a third of the rows."""
+    whose relative precision rests on that sum. 600 short rows, whose sums are
+    taken against the row max itself, and 66 of 65,536 columns, in fp32 on the
+    kernel that takes the sum in the max pass, against a reference that trails
+    the row max; a rounding of that reference that is not cancelled exactly shows
+    as a relative error up to ~3e-4 at |x| = 1e4 (an fp32 ulp of x log2(e)): a
+    form of the held-whole kernel that kept the reference in the log2 domain
+    and clamped the final rescale's exponent at 0 failed on about a third of
+    the short rows, which it took then."""
     from dataflow_lib_amd import api
     n_cols, std, shift = case
-    shape = (600, n_cols)
+    shape = (600 if n_cols <= 1000 else 66, n_cols)
     x = to_f64(to_storage(normal(791, shape, std=std) + shift, dt), dt)
     labels = rng(792).integers(0, n_cols, size=shape[0]).astype(np.uint32)
     step = 64.0 if dt == BF16 else 8.0
@@ -1007,7 +1041,7 @@ def test_fused_loss_on_short_rows_far_from_zero(hdl, dt, case):
 
 
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
-@pytest.mark.parametrize("shape", SHIFTED_SHAPES, ids=lambda s: "%dx%d" % s)
+@pytest.mark.parametrize("shape", SHIFTED_SHAPES + WHOLE_ROW_SHAPES, ids=lambda s: "%dx%d" % s)
 def test_fused_loss_keeps_small_losses(hdl, dt, shape):
     """Rows the label wins by 5 to 40 over a N(0, 1) bulk, so each loss is
     about the sum of the other columns' exp(x - x_label): from ~1e-1 down
@@ -1019,7 +1053,7 @@ def test_fused_loss_keeps_small_losses(hdl, dt, shape):
     x = normal(781, shape)
     labels = rng(782).integers(0, n_cols, size=n_rows).astype(np.uint32)
     for r in range(n_rows):
-        x[r, labels[r]] = 5.0 + 7.0 * r
+        x[r, labels[r]] = 5.0 + 7.0 * (r % 6)
     X = to_storage(x, dt)
     lo, hi, loss, mean = np.empty(shape), np.empty(shape), np.empty(n_rows), np.zeros(1)
     assert oracle().oracle_softmax_cross_entropy(dt, n_rows, n_cols, ptr(X), ptr(labels), ptr(lo), ptr(hi),
@@ -1036,7 +1070,9 @@ def test_fused_loss_keeps_small_losses(hdl, dt, shape):
     check_f32(gm, mean, rel=1e-4, what="fused mean loss, small losses")
 
 
-MARGIN_SHAPES = [(96, 128256), (96, 151936), (96, 1001)]   # register path (16-bit), streaming vector path, element path
+# held whole and 20 chunks per thread (16-bit; fp32: streamed), several waves
+# per row, and unaligned rows past 16 chunks per thread, streamed
+MARGIN_SHAPES = [(96, 128256), (96, 151936), (96, 1001), (96, 131201)]
 
 
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
@@ -1075,10 +1111,10 @@ def test_fused_loss_across_label_margins(hdl, dt, shape):
 
 
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
-@pytest.mark.parametrize("shape", SHIFTED_SHAPES, ids=lambda s: "%dx%d" % s)
+@pytest.mark.parametrize("shape", SHIFTED_SHAPES + WHOLE_ROW_SHAPES, ids=lambda s: "%dx%d" % s)
 def test_softmax_on_shifted_rows(hdl, dt, shape):
-    """fp32 rows past the register path take their softmax sum from the
-    online pass, so the shifted rows reach the softmax itself there"""
+    """streamed fp32 rows take their softmax sum from the online pass, so the
+    shifted rows reach the softmax itself there"""
     from dataflow_lib_amd import api
     n_rows, n_cols = shape
     X = shifted_logits(dt, shape, seed=741)
@@ -1091,19 +1127,26 @@ def test_softmax_on_shifted_rows(hdl, dt, shape):
     check_rounded(out, dt, pre, what="softmax, shifted rows")
 
 
+# launches that take row tickets (from the third row per workgroup on where
+# rows are held whole, from the second where they are streamed), others that
+# count rows in the loss's groups, split rows and small grids between them
+COUNTER_CASES = [(BF16, True, (1100, 32000)), (FP32, False, (700, 8000)), (BF16, False, (9, 5000)),
+                 (FP16, True, (600, 24584)), (BF16, True, (530, 151936)), (FP32, True, (3, 128)),
+                 (BF16, False, (1300, 16000)), (FP16, True, (1, 777)), (BF16, True, (1025, 4096)),
+                 (BF16, False, (700, 65552)), (FP32, True, (560, 32776)), (FP16, True, (560, 66000)), (BF16, True, (5, 66000)),
+                 (BF16, False, (300, 131201)), (FP32, False, (300, 66000)), (FP16, True, (40, 66000)), (FP16, True, (300, 164001))]
+
+
 def test_softmax_row_counter_across_launches(hdl):
-    """The 16-bit and fp32 softmax kernels hand rows past each workgroup's
-    first two out from a counter in the code object, and the last workgroup
-    of a launch resets it. Back-to-back launches of softmax and the fused op
-    in three types and shapes with more rows than two per workgroup, small
-    grids between large ones, register and streaming paths, all queued on one
-    stream with no host synchronization between them, must each match the
-    oracle (a counter left over from one launch would skip or repeat rows of
-    the next)."""
+    """The softmax kernels that walk rows hand the later ones out from a
+    counter in the code object, and the last workgroup of a launch resets it;
+    the others count rows in groups there. Back-to-back launches of softmax
+    and the fused op in three types, ticketed and not, small grids between
+    large ones, all queued on one stream with no host synchronization between
+    them, must each match the oracle (a counter left over from one launch
+    would skip or repeat rows of the next)."""
     from dataflow_lib_amd import api
-    cases = [(BF16, True, (1100, 32000)), (FP32, False, (700, 8000)), (BF16, False, (9, 5000)),
-             (FP16, True, (600, 24584)), (BF16, True, (530, 151936)), (FP32, True, (3, 128)),
-             (BF16, False, (1300, 16000)), (FP16, True, (1, 777)), (BF16, True, (1025, 4096))]
+    cases = COUNTER_CASES
     with Dev(hdl) as d:
         bufs = []
         for i, (dt, fused, shape) in enumerate(cases):
