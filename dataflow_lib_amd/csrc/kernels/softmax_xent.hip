@@ -42,6 +42,16 @@ __device__ __forceinline__ float online_rescale(float from, float to) {
 	return __builtin_amdgcn_exp2f(fminf((from - to) * SMX_LOG2E, 0.0f));
 }
 
+/* The same, applied to a sum whose reference may trail the max by up to 64, so
+ * that its terms reach e^64: the factor's root twice, since the factor itself
+ * is 0 in fp32 from 104 on, where a sum moved by up to 149 is still a normal
+ * number (bf16 rows at 1e4, a label 128 above most columns and 64 above some:
+ * losses of 1e-24 came out at 40 % of that). */
+__device__ __forceinline__ float online_move(float sum, float from, float to) {
+	const float root = __builtin_amdgcn_exp2f(fminf((from - to) * (0.5f * SMX_LOG2E), 0.0f));
+	return sum * root * root;
+}
+
 #define SMX_LN2 0.6931471805599453f
 
 /* log(1 + y) for y >= 0 in about fifteen instructions. One lane forms each
@@ -557,7 +567,7 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 					 * against moving it every chunk */
 					const bool move = cm > mref64;
 					if (__builtin_amdgcn_ballot_w64(move)) {
-						so = move ? so * online_rescale(mref, cm) : so;
+						so = move ? online_move(so, mref, cm) : so;
 						mref = move ? cm : mref;
 						mref64 = move ? cm + 64.0f : mref64;
 					}
@@ -584,7 +594,7 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 			}
 		}
 		m = cells_max(m, mslots);
-		if (SX) so *= online_rescale(mref, m);   /* sx against the row max */
+		if (SX) so = online_move(so, mref, m);   /* sx against the row max */
 #pragma unroll
 		for (int c = 0; c < MAXCH; c++) reg_barrier(xr[c]);
 

@@ -48,6 +48,7 @@ def test_softmax_test_shapes_reach_every_kernel(route, dt):
     special = {route(es, s) for s in T.SPECIAL_ROWS + T.MANY_ROWS}
     shifted = {route(es, s) for s in T.SHIFTED_SHAPES + T.WHOLE_ROW_SHAPES}
     assert plain >= every and special >= every and shifted >= every - {"wide"}
+    assert {route(es, (600 if c[0] <= 1000 else 66, c[0])) for c in T.FAR_CASES} >= {"main", "rows"} | ({"stream"} if es == 4 else set())
     assert {route(es, s) for s in T.MARGIN_SHAPES} >= {"rows", "any"} | ({"main", "long"} if es == 2 else {"stream"})
     assert route(es, (66, 128256), 0, es) == "element"
 

@@ -1000,7 +1000,7 @@ def test_fused_loss_on_shifted_rows(hdl, dt, shape):
 
 
 FAR_CASES = [(16, 1.0, -1.0e4), (16, 1.0, 1.0e4), (1000, 10.0, -1.0e4), (1000, 10.0, 1.0e4)]
-FAR_CASES += [(65536, 10.0, -1.0e4), (65536, 10.0, 1.0e4)]
+FAR_CASES += [(65536, 10.0, -1.0e4), (65536, 10.0, 1.0e4), (128256, 10.0, -1.0e4), (128256, 10.0, 1.0e4)]
 
 
 @pytest.mark.parametrize("dt", DTS, ids=dt_id)
@@ -1010,9 +1010,10 @@ def test_fused_loss_on_short_rows_far_from_zero(hdl, dt, case):
     the storage type there (8 in fp32 and fp16, 64 in bf16), so the losses
     are about the sum of the other columns' exp(x - x_label), small numbers
     whose relative precision rests on that sum. 600 short rows, whose sums are
-    taken against the row max itself, and 66 of 65,536 columns, in fp32 on the
-    kernel that takes the sum in the max pass, against a reference that trails
-    the row max; a rounding of that reference that is not cancelled exactly shows
+    taken against the row max itself, and 66 long ones on the kernels that
+    take the sum in the max pass, against a reference that trails the row max
+    (held whole: 128,256 columns in 16 bits, 65,536 in fp32; streamed: 128,256
+    in fp32); a rounding of that reference that is not cancelled exactly shows
     as a relative error up to ~3e-4 at |x| = 1e4 (an fp32 ulp of x log2(e)): a
     form of the held-whole kernel that kept the reference in the log2 domain
     and clamped the final rescale's exponent at 0 failed on about a third of
