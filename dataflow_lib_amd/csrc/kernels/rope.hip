@@ -179,9 +179,10 @@ __device__ __forceinline__ int rope_pair_of(int chunk, int head_dim, bool pow2) 
 }
 
 /* Vector path: one workgroup of ROPE_SLOT_THREADS per group of TG
- * consecutive tokens at a time (TG = rope_tokens_per_group: 2 for fp8, whose
- * rows are half as long, else 1), persistent over groups g = block,
- * block + grid, ... The group's Q rows (and K rows) are contiguous, so they
+ * consecutive tokens at a time (1 in the main kernels, or 2 for fp8 where
+ * rope_fp8_pairs holds; 2 or 4 in the "_multi" kernels, rope_tokens_per_group,
+ * for fp8 4; 1 with ROPE_WIDE_THREADS in the "_wide_rows" ones), persistent
+ * over groups g = block, block + grid, ... The group's Q rows (and K rows) are contiguous, so they
  * are addressed as one span through one buffer range (chunks past the last
  * token read zero and store nowhere); chunk c of a span belongs to token
  * c / (row chunks). The next group's Q and K chunks are loaded, and waves
@@ -447,10 +448,13 @@ __device__ __forceinline__ void rope_multi(uint64_t N, int model_dim, int head_d
 			return;
 		}
 	}
-	if (rope_tokens_per_group(n_tokens, model_dim, kv_dim, (int) sizeof(T)) == 4)
-		rope_slot<T, BWD, KV, 4, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
-	else
-		rope_slot<T, BWD, KV, 2, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
+	if constexpr (!IsFp8<T>::value) {   /* fp8: four, the main kernel takes its pairs */
+		if (rope_tokens_per_group(n_tokens, model_dim, kv_dim, (int) sizeof(T)) == 2) {
+			rope_slot<T, BWD, KV, 2, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
+			return;
+		}
+	}
+	rope_slot<T, BWD, KV, 4, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
 }
 
 #define ROPE_KERNELS(SUFFIX, T)                                                                                     \
