@@ -257,8 +257,8 @@ __device__ __forceinline__ void swiglu_bwd_fp8(long n, const TF * g, const TF * 
  * (8-byte loads). The reductions' barriers wait for LDS only (cells_max /
  * cells_sum2), so the prefetch stays in flight across them. Pieces past the
  * row end load zeros and are left out of the max and the sum; their stores
- * fall outside the row's range and store nothing. Rows are handed out as workgroups free
- * up, as in the 16-bit softmax: each workgroup's first two rows are block and
+ * fall outside the row's range and store nothing. Rows are handed out as
+ * workgroups free up, as in the 16-bit softmax: each workgroup's first two rows are block and
  * block + grid, every later one a ticket of the code object's launch-wide row
  * counter (g_smx_sched), taken by thread 0 at the top of a row for the row
  * after next and written to an LDS cell at once; the max reduction's barrier

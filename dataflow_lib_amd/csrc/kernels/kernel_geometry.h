@@ -29,7 +29,7 @@
 /* fp32 partial rows for the two-pass dW reduction (16 MiB) */
 #define RMS_DW_SCRATCH_FLOATS (4u << 20)
 
-/* softmax / cross-entropy: one workgroup per row, rows of up to
+/* softmax / cross-entropy, main kernels: one workgroup per row, rows of up to
  * SMX_THREADS * SMX_MAXCH 16-byte chunks held in registers */
 #define SMX_THREADS 1024
 #define SMX_MAXCH 16
@@ -180,16 +180,19 @@ GEOM_FN int f8_row_tpr(int n_cols) {
 /* fp8 -> 16-bit softmax, long rows (fp8_ops.hip, softmax_fp8_pf): one
  * SMX_THREADS workgroup per CU holding the row in registers (F8_PF_PIECES
  * 8-byte pieces per thread) while the next row streams in, half into LDS and
- * half into registers; rows of a multiple of 16 columns from F8_PF_MIN_COLS
- * up to 8 * F8_PF_PIECES * SMX_THREADS */
+ * half into registers; rows of a multiple of 16 columns up to
+ * 8 * F8_PF_PIECES * SMX_THREADS. smx_kernel_for sends it more than 512 rows
+ * of more than 8192 pieces; the shorter rows that reach the main kernel (2^26
+ * of them and more) are left out by F8_PF_MIN_COLS */
 #define F8_PF_PIECES 16
 #define F8_PF_MIN_COLS 32768
 GEOM_FN int f8_smx_pf_ok(int n_cols) {
 	return n_cols >= F8_PF_MIN_COLS && (n_cols % 16) == 0 && n_cols / 8 <= F8_PF_PIECES * SMX_THREADS;
 }
 
-/* softmax register-row paths: the fewest chunks per thread that a row there
- * has (smx_kernel_for sends shorter ones elsewhere) */
+/* softmax register-row paths: the fewest chunks per thread, of its own, that a
+ * row there has. The main kernels test it (smx); the "_long_rows" ones rely on
+ * smx_kernel_for. */
 GEOM_CONST int smx_regs_atleast(int elem_bytes, int maxch) {
 	return maxch > SMX_MAXCH ? SMX_MAXCH + 1 : (elem_bytes == 4 ? 6 : 8);
 }

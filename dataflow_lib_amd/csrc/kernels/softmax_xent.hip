@@ -356,12 +356,14 @@ typedef __attribute__((address_space(3))) void * lds_ptr_t;
 template <typename T, typename TO, bool FUSED, int MAXCH = SMX_MAXCH>
 __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO * out, const uint32_t * labels, float * loss) {
 	constexpr int VEC = VecOf<T>::N;
-	/* chunks per thread that every row here has: shorter ones go to other
-	 * kernels (smx_kernel_for). The first MINCH chunks go without a test of
-	 * the row's count, so those tests' masks need not be kept in (spilled)
-	 * scalar registers: bf16 fused 1024 x 100000 91.5 -> 87.1 us, softmax
-	 * 1024 x 128256 98.2 -> 95.7 us. Not in the kernels that then spilled
-	 * vector registers (fp16 softmax, and the bf16 ones of 20 chunks). */
+	/* chunks per thread, of its own, that every row here has: shorter ones go
+	 * to other kernels or paths (smx_kernel_for, smx). The mask of the lanes
+	 * past the row's end looks at no chunk before the ATLEAST-th, and the
+	 * first MINCH chunks go without a test of the row's count, so those
+	 * tests' masks need not be kept in (spilled) scalar registers: bf16 fused
+	 * 1024 x 100000 91.5 -> 87.1 us, softmax 1024 x 128256 98.2 -> 95.7 us.
+	 * MINCH is 0 in the kernels that otherwise spilled vector registers, the
+	 * fp16 softmax and the bf16 ones of 20 chunks. */
 	constexpr int ATLEAST = smx_regs_atleast((int) sizeof(T), MAXCH);
 	constexpr int MINCH = (IsF16<T>::value ? FUSED : MAXCH == SMX_MAXCH) ? ATLEAST : 0;
 	using W = SmxWord<T>;
@@ -563,7 +565,7 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 					/* the reference moves only when this lane's max passes it
 					 * by more than 64 (rare after the first chunk: a
 					 * wave-uniform branch), so the terms stay below e^64 and
-					 * 128 of them cannot overflow; measured 382.2 -> 380.8 us
+					 * MAXCH * VEC (at most 160) of them cannot overflow; measured 382.2 -> 380.8 us
 					 * against moving it every chunk */
 					const bool move = cm > mref64;
 					if (__builtin_amdgcn_ballot_w64(move)) {
@@ -636,7 +638,7 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 #pragma unroll
 		for (int c = 0; c < MAXCH; c++) {
 			__builtin_amdgcn_sched_barrier(0);
-			/* every lane issues all SMX_MAXCH stores (chunks past the row lie
+			/* every lane issues all MAXCH stores (chunks past the row lie
 			 * outside its buffer range and store nowhere), so the wait below
 			 * can count them */
 			{
@@ -666,8 +668,8 @@ __device__ __forceinline__ void smx_regs(int n_rows, int n_cols, const T * X, TO
 		}
 		/* in flight here, oldest first: the rest of the previous row's stores,
 		 * the next row's loads (issued during the max and sum passes) and
-		 * this row's SMX_MAXCH stores. Completions are in order, so waiting
-		 * until at most SMX_MAXCH remain means the next row's LDS part and
+		 * this row's MAXCH stores. Completions are in order, so waiting
+		 * until at most MAXCH remain means the next row's LDS part and
 		 * label have landed before that row reads them, while this row's
 		 * stores drain behind it; waiting before the output pass instead held
 		 * the pass up until the LDS part requested during the sum pass had
@@ -753,8 +755,9 @@ __device__ __forceinline__ void smx_stream(int n_rows, int n_cols, const T * X, 
 
 /* Rows longer than the register paths hold (more than SMX_MAXCH 16-byte
  * chunks per thread, SMX_LONG_MAXCH for 16-bit rows), 16-byte aligned, or
- * (RAGGED, kernels of their own) at any alignment that input and output share: streaming passes over the row with
- * 16-byte accesses. The first pass finds the row max and, online, the sum of
+ * (RAGGED, kernels of their own) at any alignment that input and output share,
+ * and aligned short rows that are too many for the "_rows" kernels: streaming
+ * passes over the row with 16-byte accesses. The first pass finds the row max and, online, the sum of
  * exp(x - m) over the unrounded differences (each thread keeps its running
  * max and its sum against it, rescaled when the max grows; mref = 0 while the
  * max is still -inf; the workgroup combines them against the row max). In
@@ -781,8 +784,9 @@ __device__ __forceinline__ void smx_stream_vec(int n_rows, int n_cols, const T *
 	 * the 20-chunk register path holds now: bf16 fused 660.9 -> 591.1 us,
 	 * softmax 651.1 -> 563.5 us). The outputs are bit-identical; the loss sum is rescaled
 	 * at other chunks, so a loss can differ in its last bits. RAGGED rows hold
-	 * as much, though some of their kernels then spill a few registers: with
-	 * a group less fused fp32 1024 x 128257 took 235 us instead of 220. They
+	 * as much, though their fp32 and fp16 kernels then spill (vector registers:
+	 * fp32 softmax 55, fused 103, fp16 softmax 21, fused 5): with a group less
+	 * fused fp32 1024 x 128257 took 235 us instead of 220. They
 	 * have kernels of their own because the windows' bounds made the aligned
 	 * ones spill (fused fp32 512 x 200000 167 -> 188 us). */
 	constexpr int HG = sizeof(T) == 4 ? 4 : (FUSED ? 3 : 4);
