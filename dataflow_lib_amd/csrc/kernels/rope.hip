@@ -448,13 +448,10 @@ __device__ __forceinline__ void rope_multi(uint64_t N, int model_dim, int head_d
 			return;
 		}
 	}
-	if constexpr (!IsFp8<T>::value) {   /* fp8: four, the main kernel takes its pairs */
-		if (rope_tokens_per_group(n_tokens, model_dim, kv_dim, (int) sizeof(T)) == 2) {
-			rope_slot<T, BWD, KV, 2, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
-			return;
-		}
-	}
-	rope_slot<T, BWD, KV, 4, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
+	if (IsFp8<T>::value || rope_tokens_per_group(n_tokens, model_dim, kv_dim, (int) sizeof(T)) == 4)   /* fp8: the main kernel takes its pairs */
+		rope_slot<T, BWD, KV, 4, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
+	else
+		rope_slot<T, BWD, KV, 2, ROPE_TG_QJ>(n_tokens, model_dim, head_dim, kv_dim, theta, seq_positions, X_q, X_k, kv);
 }
 
 #define ROPE_KERNELS(SUFFIX, T)                                                                                     \
