@@ -8,7 +8,7 @@
  */
 #include "rms_norm_impl.h"
 
-__device__ float g_rms_dw_partials[RMS_DW_SCRATCH_FLOATS];
+__device__ __attribute__((aligned(256))) float g_rms_dw_partials[RMS_DW_SCRATCH_FLOATS];
 /* number of partial rows written by the last main pass (its grid size) */
 __device__ int g_rms_dw_nparts;
 

@@ -96,7 +96,7 @@ __device__ __forceinline__ void waves_sum2(float & a, float & b, float * cells, 
 #define SMX_GROUPS 256
 #define SMX_GROUP_WGS 64
 #define SMX_GROUP_STRIDE 32   /* counters 128 bytes apart */
-__device__ unsigned int g_smx_group_done[(SMX_GROUPS + 1) * SMX_GROUP_STRIDE];
+__device__ __attribute__((aligned(256))) unsigned int g_smx_group_done[(SMX_GROUPS + 1) * SMX_GROUP_STRIDE];
 __device__ double g_smx_group_sum[SMX_GROUPS];
 
 struct SmxGroup {

@@ -20,7 +20,9 @@
 struct SmxSplitPart {
 	float m, sd, sx, unused;
 };
-__device__ SmxSplitPart g_smx_split[SMX_SPLIT_ROWS * SMX_SPLIT_MAX];
+/* a row's parts in two whole lines: where the compiler's placement had them in
+ * three, 16 x 128256 bf16 took 10.05 us instead of 9.87 */
+__device__ __attribute__((aligned(256))) SmxSplitPart g_smx_split[SMX_SPLIT_ROWS * SMX_SPLIT_MAX];
 __device__ float g_smx_split_xlab[SMX_SPLIT_ROWS];   /* a row's labelled logit */
 
 /* rounded differences of a chunk in the output type */

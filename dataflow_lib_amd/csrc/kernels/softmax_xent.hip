@@ -182,7 +182,7 @@ __device__ __forceinline__ void cells_sum2(float & a, float & b, float * cells) 
  * them. The two counters sit in different 128-byte lines. */
 #define SMX_TICKETS 0
 #define SMX_DONE 32
-__device__ unsigned int g_smx_sched[64];
+__device__ __attribute__((aligned(256))) unsigned int g_smx_sched[64];
 
 /* a row's loss, stored at device scope: the workgroup that sums the mean
  * loss may run on another XCD, whose L2 does not see this one's lines */
