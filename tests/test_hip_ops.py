@@ -662,9 +662,9 @@ SMX_SHAPES += [(5, 131080), (4, 65540), (3, 262144)]
 SMX_SHAPES += [(66, 131080), (65, 65540), (65, 262144), (66, 128256)]
 SMX_SHAPES += [(_ri(1, 40), _ri(1, 150000)), (_ri(1, 40), 8 * _ri(1, 16384))]
 # long rows with more rows than workgroups, so that later ones are handed out
-# by ticket: 600 x 140,000 (16-bit: 20 chunks per thread, fp32: streamed),
-# 300 x 200,000 (every type streams) and 560 x 66,000 (16-bit: held whole)
-SMX_SHAPES += [(600, 140000), (300, 200000), (560, 66000)]
+# by ticket: 600 x 140,000 (16-bit: 20 chunks per thread, fp32: streamed) and
+# 300 x 200,000 (every type streams)
+SMX_SHAPES += [(600, 140000), (300, 200000)]
 
 
 def logits(dt, shape, seed=101):
