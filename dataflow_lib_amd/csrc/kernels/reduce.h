@@ -24,11 +24,12 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 /* orders this wave's LDS writes and reads among its lanes (LDS only, so the
- * wave's global loads and stores stay in flight) */
+ * wave's global loads and stores stay in flight; a wave's LDS accesses are made
+ * in the order issued, so at wavefront scope only the compiler is held back) */
 __device__ __forceinline__ void wave_lds_sync() {
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
 	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
 template <int CTRL>

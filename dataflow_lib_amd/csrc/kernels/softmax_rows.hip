@@ -96,7 +96,7 @@ __device__ __forceinline__ void waves_sum2(float & a, float & b, float * cells, 
 #define SMX_GROUPS 256
 #define SMX_GROUP_WGS 64
 #define SMX_GROUP_STRIDE 32   /* counters 128 bytes apart */
-__device__ __attribute__((aligned(256))) unsigned int g_smx_group_done[(SMX_GROUPS + 1) * SMX_GROUP_STRIDE];
+__device__ __attribute__((aligned(4096))) unsigned int g_smx_group_done[(SMX_GROUPS + 1) * SMX_GROUP_STRIDE];
 __device__ double g_smx_group_sum[SMX_GROUPS];
 
 struct SmxGroup {
@@ -330,7 +330,7 @@ __device__ __forceinline__ void smx_rows(int n_rows, int n_cols, const T * X, TO
 	float sd = sd0 + sd1;
 	waves_sum2(sd, sx, scells, g, wave, lane);
 	if (FUSED && wave == 0 && loss) {
-		if (g == 1) wave_lds_sync();   /* the labelled logit, another lane's (g > 1: the sums' barrier) */
+		wave_lds_sync();   /* the labelled logit, another lane's where g == 1 (g > 1: the sums' barrier) */
 		if (lane == 0) store_loss(loss, row, lab_ok ? fused_loss(sx, m, xlab_cell[cell]) : __builtin_nanf(""));
 		/* a workgroup of one row counts it before the outputs, so that the
 		 * store, the count and the sums that follow it run beside them */

@@ -21,8 +21,9 @@ struct SmxSplitPart {
 	float m, sd, sx, unused;
 };
 /* a row's parts in two whole lines: where the compiler's placement had them in
- * three, 16 x 128256 bf16 took 10.05 us instead of 9.87 */
-__device__ __attribute__((aligned(256))) SmxSplitPart g_smx_split[SMX_SPLIT_ROWS * SMX_SPLIT_MAX];
+ * three, 16 x 128256 bf16 took 10.05 us instead of 9.87 (and on a page, with
+ * g_smx_group_done: fused 11.47 us on 256 bytes, 11.20 on 4096) */
+__device__ __attribute__((aligned(4096))) SmxSplitPart g_smx_split[SMX_SPLIT_ROWS * SMX_SPLIT_MAX];
 __device__ float g_smx_split_xlab[SMX_SPLIT_ROWS];   /* a row's labelled logit */
 
 /* rounded differences of a chunk in the output type */
